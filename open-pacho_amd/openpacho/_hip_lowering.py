@@ -50,6 +50,17 @@ template <typename T> __device__ __forceinline__ void pacho_store4(T* __restrict
   x[0] = v[0]; x[1] = v[1]; x[2] = v[2]; x[3] = v[3];
   *reinterpret_cast<V*>(p) = x;
 }
+// N elements at element alignment: rows of any length start anywhere. STREAM:
+// the nontemporal hint, for lines that nobody else reads.
+template <bool STREAM, int N, typename T>
+__device__ __forceinline__ void pacho_loadu(const T* __restrict__ p, T (&v)[N]) {
+  typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+  V x;
+  if constexpr (STREAM) x = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+  else x = *reinterpret_cast<const V*>(p);
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] = x[j];
+}
 template <typename T> __device__ __forceinline__ T pacho_min(T a, T b) { return a < b ? a : b; }
 template <typename T> __device__ __forceinline__ T pacho_max(T a, T b) { return a > b ? a : b; }
 __device__ __forceinline__ float pacho_min(float a, float b) {
@@ -312,50 +323,6 @@ def _reduction_index(shape, axes):
     return " + ".join(terms) or "0LL", prod(out_dims), prod(red_dims)
 
 
-def map_reduce_source(mapped_shape, axes, leaves, nodes, operation, acc_dtype):
-    index, count, reduced = _reduction_index(mapped_shape, axes)
-    chunks = max(1, -(-reduced // REDUCE_CHUNK))
-    if nodes:
-        params, lines, result = _body(mapped_shape, leaves, nodes)
-    else:  # reduction of a materialised array: the single leaf is the value
-        params, lines, result = _body(mapped_shape, leaves, [])
-    acc = ctype(acc_dtype)
-    value = f"({result} != 0)" if (nodes and nodes[-1][3].kind == "b") else result
-    params.append(f"{acc}* __restrict__ out")
-    body = "\n      ".join(lines)
-    waves = BLOCK // 64
-    source = f"""{_PRELUDE}
-extern "C" __global__ __launch_bounds__({BLOCK}) void pacho_map_reduce({", ".join(params)}) {{
-  __shared__ {acc} partial[{waves}];
-  const long long g = blockIdx.x;
-  const long long o = g / {chunks}LL, chunk = g % {chunks}LL;
-  const long long begin = chunk * {REDUCE_CHUNK}LL;
-  const long long end = begin + {REDUCE_CHUNK}LL < {reduced}LL ? begin + {REDUCE_CHUNK}LL : {reduced}LL;
-  {acc} acc = {_identity(operation, acc_dtype)};
-  for (long long r = begin + threadIdx.x; r < end; r += {BLOCK}LL) {{
-    const long long i = {index};
-    {{
-      {body}
-      acc = {_combine(operation, acc_dtype, "acc", f"({acc})({value})")};
-    }}
-  }}
-#pragma unroll
-  for (int offset = 1; offset < 64; offset <<= 1) {{
-    const {acc} other = __shfl_xor(acc, offset, 64);
-    acc = {_combine(operation, acc_dtype, "acc", "other")};
-  }}
-  if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {{
-    {acc} total = partial[0];
-    for (int w = 1; w < {waves}; ++w) total = {_combine(operation, acc_dtype, "total", "partial[w]")};
-    out[g] = total;
-  }}
-}}
-"""
-    return source, count, chunks
-
-
 def _leaf_of(node):
     return _Leaf(node.op == "scalar", node.dtype, node.shape)
 
@@ -418,18 +385,20 @@ class HIPLowering:
         if prod(mapped.shape) > 2**31 - 1:
             raise ValueError("Array exceeds GPU indexing limits")
         specs, nodes = _graph(group, leaves)
-        source, count, chunks = map_reduce_source(
+        from ._hip_map_reduce import map_reduce_source  # it builds on this module's sources
+
+        payload = map_reduce_source(
             mapped.shape, tuple(node.attrs["axes"]), specs, nodes, operation, np.dtype(node.dtype)
         )
-        return tuple(leaves), (source, count, chunks)
+        return tuple(leaves), payload
 
     def run_map_reduce(self, node, payload, arguments, operands):
-        source, count, chunks = payload
-        out = self.backend.empty((count, chunks), node.dtype)
-        self.backend._launch(source, "pacho_map_reduce", count * chunks, operands, out)
+        source, _, chunks = payload
+        out = self.backend.empty(payload.partials, node.dtype)
+        self.backend._launch(source, "pacho_map_reduce", payload.grid, operands, out)
         if chunks == 1:
             return out
-        partial = ndarray._wrap(out, (count, chunks), node.dtype, self.backend)
+        partial = ndarray._wrap(out, payload.partials, node.dtype, self.backend)
         options = {"operation": node.attrs["operation"]} if "operation" in node.attrs else {}
         return self.backend.reduce(partial, (1,), False, node.dtype, **options)
 

@@ -1,0 +1,109 @@
+"""Mapped reductions at the edges of their kernels: rows around one vector
+group, one wave's share, the whole-workgroup rule and a chunk; columns around
+the vector width, a column block and a rows-per-step count; every way a leaf
+may be broadcast. Elements are small integers, so that every order of a sum
+gives the same value and the comparison is exact; one case per kernel checks
+that a compiled sum rounds like the eager one and stays within the bound of
+its summation order on ordinary values.
+"""
+
+import numpy as np
+import pytest
+
+import openpacho as p
+from openpacho._hip_map_reduce import BLOCK, _column_plan, map_reduce_source
+from openpacho._hip_lowering import _Leaf
+
+# (shape, reduced axes)
+ROWS = [((5, n), (1,)) for n in (1, 3, 4, 5, 63, 64, 65, 1008, 1025, 8191, 8192, 8197)]
+ROWS += [((4097, 1030), (1,)), ((4096, 1030), (1,)), ((3, 5, 67), (1, 2)), ((100000,), (0,)), ((70001, 3), (1,))]
+COLUMNS = [((n, 5), (0,)) for n in (1, 7, 8, 9, 4099)] + [((300, n), (0,)) for n in (2, 3, 4, 63, 1023, 1024, 1025, 1028)]
+COLUMNS += [((3, 50, 6), (1,)), ((2, 7, 5, 11), (1, 2)), ((20011, 257), (0,)), ((513, 1, 9), (0,))]
+OTHER = [((6, 31, 7), (0, 2)), ((0, 4), (0,)), ((3, 1), (0,))]
+
+
+def _leaf_shapes(shape):
+    """Second operands of every broadcast kind of `shape`."""
+    ones = (1,) * len(shape)
+    kinds = {shape, ones, shape[-1:], shape[:-1] + (1,), shape[:1] + ones[1:]}
+    if len(shape) > 2:
+        kinds.add((1, shape[1]) + ones[2:])
+    return sorted(kinds)
+
+
+CASES = [(shape, axes, i) for i, (shape, axes) in enumerate(ROWS + COLUMNS + OTHER)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,axes,index", CASES)
+def test_mapped_reductions_are_exact_on_small_integers(hip, shape, axes, index):
+    # Types, operations and broadcast kinds rotate over the shapes.
+    rng = np.random.default_rng(index)
+    kinds = _leaf_shapes(shape)
+    for turn in range(2):
+        dtype = (np.float32, np.float64, np.int32)[(index + turn) % 3]
+        name = "sum" if turn == 0 or not np.prod(shape) else ("min", "max")[index % 2]
+        host = rng.integers(-3, 4, shape).astype(dtype)
+        other = rng.integers(-3, 4, kinds[(index + turn * 2) % len(kinds)]).astype(dtype)
+        function = getattr(np, name)
+        compiled = p.compile(lambda x, b: function(x * b - 2, axis=axes))
+        got = p.asnumpy(compiled(p.asarray(host, backend=hip), p.asarray(other, backend=hip)))
+        np.testing.assert_array_equal(got, function(host * other - 2, axis=axes))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,axis", [((37, 5000), 1), ((9000, 49), 1), ((3, 20000), 1), ((20000, 129), 0)])
+def test_mapped_sums_round_like_the_eager_sum_and_within_their_bound(hip, shape, axis):
+    host = np.random.default_rng(1).standard_normal(shape).astype(np.float32)
+    x = p.asarray(host, backend=hip)
+    got = p.asnumpy(p.compile(lambda x: np.sum(x * 1.5, axis=axis))(x))
+    mapped = host * np.float32(1.5)
+    if axis == 1:
+        np.testing.assert_array_equal(got, p.asnumpy(np.sum(x * 1.5, axis=axis)))
+    exact = mapped.astype(np.float64).sum(axis=axis)
+    # Recursive summation: depth * u * sum |x|. The longest chain of additions
+    # is a thread's rows / 8 or 32 vector groups, then the trees and the merge
+    # of the partials: below 160 for these shapes.
+    bound = 160 * 2.0**-24 * np.abs(mapped.astype(np.float64)).sum(axis=axis)
+    assert np.all(np.abs(got - exact) <= bound)
+
+
+@pytest.mark.gpu
+def test_extrema_of_mapped_rows_and_columns_keep_nan_infinities_and_signed_zeros(hip):
+    host = np.full((70, 69), 5, np.float32)
+    host[3, 68], host[10, 1], host[20, 40], host[30, 5] = np.nan, np.inf, -np.inf, 0.0
+    host[40], host[41] = 0.0, -0.0
+    host[41, 68] = 0.0
+    x = p.asarray(host, backend=hip)
+    for axis in (0, 1):
+        for name in ("min", "max"):
+            function = getattr(np, name)
+            got = p.asnumpy(p.compile(lambda x: function(-x, axis=axis))(x))
+            want = p.asnumpy(getattr(p, name)(-x, axis=axis))
+            np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+            with np.errstate(invalid="ignore"):
+                np.testing.assert_array_equal(got, function(-host, axis=axis))
+
+
+@pytest.mark.parametrize("width", [2, 4])
+def test_column_plans_cover_every_element_once(width):
+    rng = np.random.default_rng(width)
+    sizes = [1, 2, 3, 15, 16, 17, 255, 256, 257, 1025, 4096, 100003]
+    for outer, reduced, inner in [(int(a), int(b), int(c)) for a, b, c in rng.choice(sizes, (400, 3))]:
+        across, blocks, step, rows, chunks = _column_plan(outer, reduced, inner, width, 8)
+        groups = -(-inner // width)
+        assert across * step <= BLOCK and (blocks - 1) * across < groups <= blocks * across
+        assert rows % step == 0 and (chunks - 1) * rows < reduced <= chunks * rows
+
+
+@pytest.mark.parametrize("shape,axes", [((8, 100, 12), (1,)), ((8, 3, 12), (0, 2)), ((5, 8193), (1,))])
+@pytest.mark.parametrize("operation,dtype", [("sum", "f8"), ("min", "u8"), ("max", "?")])
+def test_sources_compile(shape, axes, operation, dtype):
+    from test_abi import _compiles
+
+    dtype = np.dtype(dtype)
+    leaves = [_Leaf(False, dtype, shape), _Leaf(False, dtype, shape[-1:]), _Leaf(True, dtype, ())]
+    op = "where" if dtype.kind != "b" else "equal"
+    nodes = [(op, [0, 1, 2][: 3 if op == "where" else 2], (dtype,) * 3, dtype)]
+    status, log = _compiles(map_reduce_source(shape, axes, leaves, nodes, operation, dtype)[0])
+    assert status == 0, log
