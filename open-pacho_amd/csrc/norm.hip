@@ -142,32 +142,115 @@ __device__ __forceinline__ Pair<T> registers_to_pair(const T (&v)[N]) {
 //   kFinal   one chunk per row: write the row's norm;
 //   kPairs   several rows of several chunks: one pair per unit;
 //   kRunning a single row: every wave folds its chunks into a running pair
-//            and each workgroup writes one pair (few pairs left to merge).
-constexpr int kFinal = 0, kPairs = 1, kRunning = 2;
+//            and each workgroup writes one pair (few pairs left to merge);
+//   kWalk    rows of several chunks, enough of them to keep the chip's waves
+//            busy one row each: a wave folds its row's chunks in order and
+//            writes the norm (no pairs in memory, no merge launch; 16384 rows
+//            of 8190 float32: 146 -> 84 us).
+// kVector: nearly every chunk is whole and 16-byte aligned (65536 rows of 4096
+// float32: 154 us; the guarded loads of the other form 168 us). Otherwise a
+// wave reads groups of 16 bytes at element alignment, all of a chunk's before
+// the first is used (22544 rows of 3547: 61 us element by element, 48 us like
+// this); rows of up to half a chunk take half the loads
+// (LOADS = kLoads / 2), so that short rows do not pay for empty registers.
+constexpr int kFinal = 0, kPairs = 1, kRunning = 2, kWalk = 3;
+// Rows at which kWalk gives every compute unit 16 waves.
+constexpr int64_t kWalkRows = 4096;
+// Longest row of norm_short_kernel: 16 elements a lane of one wave.
+constexpr int64_t kShort = 1024;
 
-template <typename T, bool kVector, int MODE>
+// The `len` elements at `base`, `lanes` lanes taking a group of 16 bytes each
+// in turn; the last len % width elements, one a lane, come in v's last entry.
+// Entries past the end are +0, which changes neither the max nor the sum.
+// STREAM: nontemporal loads, for waves that read whole lines of one row; short
+// rows share lines with the rows of other waves.
+template <typename T, int LOADS, bool STREAM>
+__device__ __forceinline__ void load_chunk(const T* base, int64_t len, int lane, int lanes,
+                                           T (&v)[LOADS * Traits<T>::width + 1]) {
+  constexpr int W = Traits<T>::width;
+  typedef T V __attribute__((ext_vector_type(W), aligned(sizeof(T))));
+  const int groups = int(len / W), rest = int(len % W);
+  const auto load = [&](int at) -> V {
+    const V* p = reinterpret_cast<const V*>(base) + at;
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+  };
+  V q[LOADS];
+  v[LOADS * W] = T(0);
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    q[i] = V(T(0));
+    if (i * lanes + lane < groups) q[i] = load(i * lanes + lane);
+  }
+  if (lane < rest) v[LOADS * W] = base[int64_t(groups) * W + lane];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i)
+#pragma unroll
+    for (int w = 0; w < W; ++w) v[i * W + w] = q[i][w];
+}
+
+// Short rows (up to kShort elements): `lanes` lanes of a wave share a row,
+// about 16 elements each, so that a wave handles 64 / lanes rows at once and
+// no lane holds more empty registers than values. A wave per row took 1460 us
+// for 1200000 rows of 49 float32 and 746 us for 600000 rows of 230; like
+// this 50 and 89 us. The pair is formed without branches, as
+// lane_pair below does: a NaN makes the sum NaN whatever the max was, then a
+// max of +inf or 0 decides.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void norm_short_kernel(const T* __restrict__ x, T* __restrict__ out,
+                                                            int64_t outer, int64_t reduced, int lanes) {
+  constexpr int LOADS = 16 / Traits<T>::width;
+  constexpr int N = LOADS * Traits<T>::width + 1;
+  const int lane = threadIdx.x & (lanes - 1);
+  const int64_t o = int64_t(blockIdx.x) * (kBlock / lanes) + threadIdx.x / lanes;
+  T v[N];
+  load_chunk<T, LOADS, false>(x + (o < outer ? o : 0) * reduced, o < outer ? reduced : 0, lane, lanes, v);
+  T m = T(0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) m = dmax(m, dabs(v[i]));
+  for (int off = lanes / 2; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off, 64));
+  const int e = dexponent(m);
+  T t = T(0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const T s = dldexp(v[i], -e);
+    t = dfma(s, s, t);
+  }
+  for (int off = lanes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  Pair<T> p = {T(e), t};
+  if (isnan(t)) p = {T(NAN), T(0)};
+  else if (isinf(m)) p = {T(INFINITY), T(0)};
+  else if (m == T(0)) p = {T(-INFINITY), T(0)};
+  if (lane == 0 && o < outer) out[o] = finish(p);
+}
+
+template <typename T, int LOADS, bool kVector, int MODE>
 __global__ __launch_bounds__(kBlock) void norm_rows_kernel(const T* __restrict__ x, T* __restrict__ out,
                                                            int64_t outer, int64_t reduced, int64_t chunks) {
   using V = typename Traits<T>::V;
   constexpr int W = Traits<T>::width;
-  constexpr int N = kLoads * W;
+  constexpr int N = LOADS * W + (kVector ? 0 : 1);
+  constexpr int64_t kLen = int64_t(64) * LOADS * W;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t units = outer * chunks;
+  const int64_t units = MODE == kWalk ? outer : outer * chunks;
   const int64_t stride = int64_t(gridDim.x) * (kBlock / 64);
   Pair<T> running = {T(-INFINITY), T(0)};
-  for (int64_t g = int64_t(blockIdx.x) * (kBlock / 64) + wave; g < units; g += stride) {
-    const int64_t o = g / chunks, ch = g - o * chunks;
-    const int64_t begin = ch * chunk_len<T>();
-    const int64_t len = reduced - begin < chunk_len<T>() ? reduced - begin : chunk_len<T>();
+  int64_t walked = 0;  // chunks of the current row already in `running` (kWalk)
+  for (int64_t g = int64_t(blockIdx.x) * (kBlock / 64) + wave; g < units;) {
+    const int64_t o = MODE == kWalk ? g : g / chunks, ch = MODE == kWalk ? walked : g - o * chunks;
+    const int64_t begin = ch * kLen;
+    const int64_t len = reduced - begin < kLen ? reduced - begin : kLen;
     const T* base = x + o * reduced + begin;
     T v[N];
-    if (kVector && len == chunk_len<T>()) {
+    if constexpr (!kVector) {
+      load_chunk<T, LOADS, true>(base, len, lane, 64, v);
+    } else if (len == kLen) {
       const V* bv = reinterpret_cast<const V*>(base);
-      V q[kLoads];
+      V q[LOADS];
 #pragma unroll
-      for (int i = 0; i < kLoads; ++i) q[i] = __builtin_nontemporal_load(bv + i * 64 + lane);
+      for (int i = 0; i < LOADS; ++i) q[i] = __builtin_nontemporal_load(bv + i * 64 + lane);
 #pragma unroll
-      for (int i = 0; i < kLoads; ++i)
+      for (int i = 0; i < LOADS; ++i)
 #pragma unroll
         for (int w = 0; w < W; ++w) v[i * W + w] = q[i][w];
     } else {
@@ -178,7 +261,13 @@ __global__ __launch_bounds__(kBlock) void norm_rows_kernel(const T* __restrict__
       }
     }
     const Pair<T> p = registers_to_pair<T, N>(v);
-    if (MODE == kRunning) {
+    if (MODE == kWalk) {
+      running = merge(running, p);
+      if (++walked < chunks) continue;
+      if (lane == 0) out[o] = finish(running);
+      running = {T(-INFINITY), T(0)};
+      walked = 0;
+    } else if (MODE == kRunning) {
       running = merge(running, p);
     } else if (lane == 0) {
       if (MODE == kFinal) {
@@ -188,6 +277,7 @@ __global__ __launch_bounds__(kBlock) void norm_rows_kernel(const T* __restrict__
         out[2 * g + 1] = p.t;
       }
     }
+    g += stride;
   }
   if (MODE == kRunning) {
     __shared__ T ks[kBlock / 64], ts[kBlock / 64];
@@ -340,9 +430,11 @@ struct Workspace {
 
 struct RowPlan {
   int mode = kFinal;
-  bool vector = false;
+  bool vector = false;  // nearly all chunks whole and aligned
+  int lanes = 0;        // lanes per row of norm_short_kernel, 0 for norm_rows_kernel
   int64_t chunks = 0, grid = 0;
-  int64_t pairs = 0;   // pairs the row pass writes (0 in kFinal mode)
+  int64_t pairs = 0;   // pairs the row pass writes (0 in the modes that write norms)
+  int64_t claimed = 0; // pairs of a pass over units: hp_norm_noalloc's measure of a shape
   int64_t second = 0;  // pairs the first merge pass writes when it is not the last
 };
 
@@ -350,19 +442,27 @@ template <typename T>
 RowPlan plan_rows(hp_ctx* ctx, const T* x, int64_t outer, int64_t reduced) {
   RowPlan plan;
   plan.chunks = hp::ceil_div(reduced, chunk_len<T>());
-  const int64_t units = outer * plan.chunks;
-  plan.vector = reinterpret_cast<uintptr_t>(x) % 16 == 0 && (reduced * int64_t(sizeof(T))) % 16 == 0;
-  plan.mode = plan.chunks == 1 ? kFinal : (outer == 1 ? kRunning : kPairs);
+  if (reduced <= kShort) {
+    plan.lanes = Traits<T>::width;  // load_chunk's last elements take a lane each
+    while (plan.lanes < 64 && plan.lanes * 16 < reduced) plan.lanes *= 2;
+    plan.grid = hp::ceil_div(outer, kBlock / plan.lanes);
+    hp::require(plan.grid <= hp::kMaxGrid, "too many rows for one launch");
+    return plan;
+  }
+  plan.vector = reinterpret_cast<uintptr_t>(x) % 16 == 0 && (reduced * int64_t(sizeof(T))) % 16 == 0 &&
+                (reduced % chunk_len<T>() == 0 || plan.chunks > 8);
+  plan.mode = plan.chunks == 1 ? kFinal : (outer == 1 ? kRunning : (outer >= kWalkRows ? kWalk : kPairs));
+  const int64_t units = plan.mode == kWalk ? outer : outer * plan.chunks;
   // Enough resident waves to keep HBM busy; the grid loops over the rest.
   const int64_t resident = int64_t(ctx->compute_units) * kResidentGroupsPerCU;
   plan.grid = hp::ceil_div(units, kBlock / 64);
   if (plan.grid > resident) plan.grid = resident;
-  if (plan.mode != kFinal) {
-    const int64_t per_row = plan.mode == kRunning ? plan.grid : plan.chunks;
-    plan.pairs = plan.mode == kRunning ? plan.grid : units;
-    const int64_t groups = hp::ceil_div(per_row, kMerge);
-    plan.second = groups > 1 ? outer * groups : 0;
-  }
+  if (plan.mode == kFinal) return plan;
+  const int64_t per_row = plan.mode == kRunning ? plan.grid : plan.chunks;
+  const int64_t groups = hp::ceil_div(per_row, kMerge);
+  plan.claimed = plan.mode == kRunning ? plan.grid : outer * plan.chunks;
+  plan.second = groups > 1 ? outer * groups : 0;
+  if (plan.mode != kWalk) plan.pairs = plan.claimed;
   return plan;
 }
 
@@ -370,21 +470,27 @@ template <typename T>
 void run_rows(hp_ctx* ctx, const RowPlan& plan, const T* x, T* out, int64_t outer, int64_t reduced,
               Workspace ws) {
   const int64_t grid = plan.grid, chunks = plan.chunks;
-  T* target = plan.mode == kFinal ? out : static_cast<T*>(ws.first);
-#define PACHO_NORM_LAUNCH(VEC, MODE_)                                                                           \
-  norm_rows_kernel<T, VEC, MODE_><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks)
-  if (plan.vector) {
-    if (plan.mode == kFinal) PACHO_NORM_LAUNCH(true, kFinal);
-    else if (plan.mode == kRunning) PACHO_NORM_LAUNCH(true, kRunning);
-    else PACHO_NORM_LAUNCH(true, kPairs);
-  } else {
-    if (plan.mode == kFinal) PACHO_NORM_LAUNCH(false, kFinal);
-    else if (plan.mode == kRunning) PACHO_NORM_LAUNCH(false, kRunning);
-    else PACHO_NORM_LAUNCH(false, kPairs);
+  if (plan.lanes > 0) {
+    norm_short_kernel<T><<<grid, kBlock, 0, ctx->stream>>>(x, out, outer, reduced, plan.lanes);
+    hp::check_launch("norm_short");
+    return;
   }
+  const bool direct = plan.mode == kFinal || plan.mode == kWalk;
+  T* target = direct ? out : static_cast<T*>(ws.first);
+#define PACHO_NORM_LAUNCH(MODE_)                                                                                 \
+  do {                                                                                                          \
+    if (plan.vector) norm_rows_kernel<T, kLoads, true, MODE_><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks); \
+    else norm_rows_kernel<T, kLoads, false, MODE_><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks);            \
+  } while (0)
+  if (plan.mode == kFinal && reduced <= chunk_len<T>() / 2)
+    norm_rows_kernel<T, kLoads / 2, false, kFinal><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks);
+  else if (plan.mode == kFinal) PACHO_NORM_LAUNCH(kFinal);
+  else if (plan.mode == kRunning) PACHO_NORM_LAUNCH(kRunning);
+  else if (plan.mode == kWalk) PACHO_NORM_LAUNCH(kWalk);
+  else PACHO_NORM_LAUNCH(kPairs);
 #undef PACHO_NORM_LAUNCH
   hp::check_launch("norm_rows");
-  if (plan.mode == kFinal) return;
+  if (direct) return;
   // Pair modes always finish with at least one merge pass (it writes `out`).
   T* source = static_cast<T*>(ws.first);
   T* spare = static_cast<T*>(ws.second);
@@ -420,7 +526,7 @@ void run_norm(hp_ctx* ctx, const T* x, T* out, int64_t outer, int64_t reduced, i
   const RowPlan plan = plan_rows<T>(ctx, x, outer, reduced);
   Workspace ws;
   if (plan.pairs > 0) ws.first = hp::scratch_alloc(ctx, size_t(plan.pairs) * 2 * sizeof(T));
-  if (plan.second > 0) ws.second = hp::scratch_alloc(ctx, size_t(plan.second) * 2 * sizeof(T));
+  if (plan.pairs > 0 && plan.second > 0) ws.second = hp::scratch_alloc(ctx, size_t(plan.second) * 2 * sizeof(T));
   run_rows<T>(ctx, plan, x, out, outer, reduced, ws);
   if (ws.second) hp::scratch_free(ctx, ws.second);
   if (ws.first) hp::scratch_free(ctx, ws.first);
@@ -490,7 +596,9 @@ void run_norm_noalloc(hp_ctx* ctx, const T* x, T* out, int64_t outer, int64_t re
     return run_cols<T>(ctx, plan, x, out, outer, reduced, inner, buffers);
   }
   const RowPlan plan = plan_rows<T>(ctx, x, outer, reduced);
-  const size_t first = align_up(size_t(plan.pairs) * 2 * sizeof(T));
+  // Shapes are refused by the pairs of their units also where the kernel chosen
+  // writes none, so that which shapes fit does not depend on that choice.
+  const size_t first = align_up(size_t(plan.claimed) * 2 * sizeof(T));
   const size_t second = size_t(plan.second) * 2 * sizeof(T);
   check_scratch(first, second);
   Workspace ws;
