@@ -6,6 +6,7 @@
 #include <algorithm>
 
 #include "gemm.h"
+#include "gemm_direct.h"
 
 namespace {
 
@@ -17,6 +18,11 @@ __global__ __launch_bounds__(256) void zero_kernel(T* __restrict__ out, int64_t 
 // Products of every layout: C[b] = op(A[b']) @ op(B[b'']).
 void run(hp_ctx* ctx, int dtype, bool ta, bool tb, const void* a, const void* b, void* c, int64_t m, int64_t n,
          int64_t k, const hpgemm::BatchDesc& bd, int64_t batch) {
+  const hpgemm::DirectPlan direct = hpgemm::direct_plan(ctx->compute_units, dtype, m, n, k, batch);
+  if (direct.fi > 0) {
+    (dtype == HP_F32 ? hpgemm::direct_f32 : hpgemm::direct_f64)(ctx, direct, ta, tb, a, b, c, m, n, k, bd, batch);
+    return;
+  }
   static const hpgemm::Run table[2][4] = {
       {hpgemm::f32_nn, hpgemm::f32_tn, hpgemm::f32_nt, hpgemm::f32_tt},
       {hpgemm::f64_nn, hpgemm::f64_tn, hpgemm::f64_nt, hpgemm::f64_tt},
@@ -102,6 +108,95 @@ void run_int(hp_ctx* ctx, int dtype, const void* a, const void* b, void* c, int6
 }
 
 }  // namespace
+
+namespace {
+
+// Whether the direct kernels take a product: where the LDS-staged tiles of
+// gemm_kernels.h are mostly padding or too few for the chip. The direct kernels
+// reach 55-65% of the MFMA rate whatever the shape; the staged ones 80-95% of
+// it on large whole tiles, little where tiles are cut, and the fp64 ones need
+// 256 x 128 outputs per workgroup. Lines between measurements on one MI355X, us
+// staged / direct:
+//   fp32, padding of the staged tiles (128 x 128, or 256 x 256 for more than
+//   256 slices) over 40%: 16 x 8192 x 8192 (m, n, k) 273 / 47, 128 x 8192 x 8192
+//   274 / 157, 202 x (29 x 18 x 936) 71 / 17; over 15%: 700 x 700 x 3000 49 / 34,
+//   56 x (592 x 429 x 173) 100 / 99, 400 x 4000 x 2000 (3.2e9) 78 / 86; up to one
+//   and a half 64 x 64 tiles per compute unit: 1000^3 33 / 25, 512 x 512 x 8192
+//   70 / 54, 1200 x 1200 x 2000 (2.9e9) 64 / 64; else 1000 x 3000 x 333 35 / 39,
+//   2500 x 2500 x 100 23 / 35. Products of the narrow kernel's extents stay
+//   there (1024^3 21 / 24, 8 x 512^3 21 / 30).
+//   fp64: 560 x 453 x 688 56 / 17, 1024^3 60 / 42, 2048 x 2048 x 256 65 / 57,
+//   8192 x 128 x 8192 575 / 291; large products 1200 x 1200 x 2000 125 / 133,
+//   2048^3 277 / 299; their kernel for any K (no multiple of 16) 1500^3
+//   168 / 142, 2672 x 2528 x 675 about even; few slices in many tiles 3025 x 2024
+//   x 75 33 / 55.
+bool direct_serves(int64_t cus, int dtype, int64_t m, int64_t n, int64_t k, int64_t batch) {
+  const double work = double(m) * double(n) * double(k) * double(batch);
+  const int64_t slices = hp::ceil_div(k, 16);
+  const double tiles64 = double(hp::ceil_div(m, 64)) * double(hp::ceil_div(n, 64)) * double(batch);
+  const auto fill = [&](int64_t bm, int64_t bn) {
+    return double(m) * double(n) / (double(hp::ceil_div(m, bm) * bm) * double(hp::ceil_div(n, bn) * bn));
+  };
+  if (dtype == HP_F64) {
+    if (slices <= 8 && tiles64 > 2.0 * cus) return false;
+    return fill(256, 128) < 0.6 || work <= 2.4e9 || (k % 16 != 0 && slices >= 64 && work <= 8e9);
+  }
+  const bool narrow = m % 64 == 0 && n % 64 == 0 && k % 16 == 0 && tiles64 >= cus && tiles64 <= 4.0 * cus &&
+                      work <= double(cus) * double(1 << 23);
+  if (narrow) return false;
+  const double filled = slices > 256 ? fill(256, 256) : fill(128, 128);
+  if (filled < 0.6) return work <= 9e9;
+  if (filled < 0.85) return work <= 2.6e9;
+  return tiles64 <= 1.5 * cus && work <= 2.2e9;
+}
+
+}  // namespace
+
+// Tile and K split by the time they would take: a compute unit works off its
+// workgroups' tiles one after the other, each wave a quarter of the slices, so
+// a candidate costs (workgroups per compute unit, rounded up) x (MFMA blocks of
+// the tile) x (slices per wave), over the share of the MFMA rate its loads let
+// it reach, and a split the second kernel. `rate` and the overheads are fitted
+// to sweeps of every tile and split over 24 shapes in both types; the choice
+// was the fastest or within 6% of it on all but two.
+hpgemm::DirectPlan hpgemm::direct_plan(int compute_units, int dtype, int64_t m, int64_t n, int64_t k, int64_t batch) {
+  struct Candidate {
+    int fi, fj;
+    double rate;
+  };
+  static constexpr Candidate kCandidates[] = {{4, 4, 1.0},  {2, 4, 0.95}, {4, 2, 0.95}, {2, 2, 0.9},
+                                              {1, 4, 0.75}, {4, 1, 0.75}, {1, 1, 0.5}};
+  constexpr double kTile = 0.3, kSplit = 4.0;  // us: a workgroup's start and store; the second kernel
+  DirectPlan best;
+  if (!direct_serves(compute_units, dtype, m, n, k, batch)) return best;
+  double least = 0;
+  const int64_t slices = hp::ceil_div(k, 16);
+  const double unit = dtype == HP_F32 ? 0.053 : 0.107;  // us: one block over one slice
+  for (const Candidate& c : kCandidates) {
+    // Tiles move inside the operands, which only one-block extents may undercut.
+    if ((c.fi > 1 && m < 16 * c.fi) || (c.fj > 1 && n < 16 * c.fj)) continue;
+    DirectPlan p;
+    p.fi = c.fi;
+    p.fj = c.fj;
+    p.tiles_m = hp::ceil_div(m, 16 * c.fi);
+    p.tiles_n = hp::ceil_div(n, 16 * c.fj);
+    p.tiles = p.tiles_m * p.tiles_n * batch;
+    p.slices = slices;
+    for (int64_t splits = 1; splits <= 32; splits *= 2) {
+      if (splits > 1 && (slices < 16 * splits || p.tiles * splits > 4 * int64_t(compute_units))) break;
+      p.per_split = hp::ceil_div(slices, splits);
+      p.splits = hp::ceil_div(slices, p.per_split);
+      const double rounds = double(hp::ceil_div(p.tiles * p.splits, compute_units));
+      const double cost = rounds * (c.fi * c.fj * unit / c.rate * double(hp::ceil_div(p.per_split, 4)) + kTile) +
+                          (p.splits > 1 ? kSplit : 0.0);
+      if (best.fi == 0 || cost < least) {
+        best = p;
+        least = cost;
+      }
+    }
+  }
+  return best;
+}
 
 using hp::guarded;
 using hp::require;
