@@ -348,9 +348,13 @@ class ExecutionPlan:
         scope = getattr(backend, "execution_scope", None)
         launches = sum(getattr(s.payload, "dispatch_count", 1) if s.kind == "padded_matmul" else 1 for s in self.steps)
         self._execution_scope = scope if launches >= getattr(backend, "execution_scope_min_steps", 0) else None
-        # Reads of each value by later steps and by the result: a value is
+        # What runs: the steps, or the launches that the lowerer regroups them
+        # into (the steps stay what the plan is explained by).
+        arrange = getattr(self.lowering, "arrange", None)
+        self._launches = self.steps if arrange is None else arrange(self.steps, outputs)
+        # Reads of each value by later launches and by the result: a value is
         # released when the count reaches zero.
-        self._reads = Counter(id(arg) for step in self.steps for arg in step.args)
+        self._reads = Counter(id(arg) for step in self._launches for arg in step.args)
         self._reads.update(id(o) for o in outputs)
         self._executors = {
             "fused": self._run_fused,
@@ -398,8 +402,20 @@ class ExecutionPlan:
                 values[id(node)] = self._leaf(node, bindings)
             return values[id(node)]
 
-        for node, kind, args, payload in self.steps:
-            operands = [value_of(a) for a in args]
+        def release(args):
+            for arg in args:
+                reads[id(arg)] -= 1
+                if not reads[id(arg)]:
+                    values.pop(id(arg), None)
+
+        for step in self._launches:
+            operands = [value_of(a) for a in step.args]
+            if not isinstance(step, Step):  # several values of one launch
+                for node, data in zip(step.nodes, self.lowering.run_launch(step.nodes, step.payload, operands)):
+                    values[id(node)] = ndarray._wrap(data, node.shape, node.dtype, self.backend)
+                release(step.args)
+                continue
+            node, kind, args, payload = step
             if kind in ELEMENTWISE:
                 data = self._run_elementwise(node, kind, operands)
             elif kind in ("fused", "map_reduce"):
@@ -410,10 +426,7 @@ class ExecutionPlan:
                     raise NotImplementedError(f"No execution rule for {kind}")
                 data = executor(node, payload, [self._materialized(v) for v in operands])
             values[id(node)] = ndarray._wrap(data, node.shape, node.dtype, self.backend)
-            for arg in args:
-                reads[id(arg)] -= 1
-                if not reads[id(arg)]:
-                    values.pop(id(arg), None)
+            release(args)
         results = tuple(self._materialized(value_of(o)) for o in self.outputs)
         return results if self.multiple else results[0]
 

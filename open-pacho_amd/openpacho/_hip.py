@@ -219,7 +219,8 @@ class HIPBackend:
             lib_.check(self._lib, self._free(self._ctx, ptr), "hp_free")
 
     def _launch(self, source, name, grid, operands, out):
-        """Compile (cached) and launch an RTC kernel over operands + out."""
+        """Compile (cached) and launch an RTC kernel over operands + out (one
+        storage or a list of them)."""
         with self._active():
             kernel = self._kernels.get(source)
             if kernel is None:
@@ -237,7 +238,8 @@ class HIPBackend:
                     values.append(_C_SCALARS[operand.dtype](operand._data.item()))
                 else:
                     values.append(ctypes.c_void_p(operand._data.ptr))
-            values.append(ctypes.c_void_p(out.ptr))
+            for storage in out if isinstance(out, list) else (out,):
+                values.append(ctypes.c_void_p(storage.ptr))
             pointers = (ctypes.c_void_p * len(values))(*(ctypes.addressof(v) for v in values))
             self._call("hp_rtc_launch", kernel, grid, BLOCK, 0, pointers)
 

@@ -61,6 +61,13 @@ __device__ __forceinline__ void pacho_loadu(const T* __restrict__ p, T (&v)[N]) 
 #pragma unroll
   for (int j = 0; j < N; ++j) v[j] = x[j];
 }
+template <int N, typename T> __device__ __forceinline__ void pacho_storeu(T* __restrict__ p, const T (&v)[N]) {
+  typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+  V x;
+#pragma unroll
+  for (int j = 0; j < N; ++j) x[j] = v[j];
+  *reinterpret_cast<V*>(p) = x;
+}
 template <typename T> __device__ __forceinline__ T pacho_min(T a, T b) { return a < b ? a : b; }
 template <typename T> __device__ __forceinline__ T pacho_max(T a, T b) { return a > b ? a : b; }
 __device__ __forceinline__ float pacho_min(float a, float b) {
@@ -214,8 +221,9 @@ def _body(root_shape, leaves, nodes, var="i", leaf_value=None, suffix="LL"):
     return params, lines, names[-1]
 
 
-def elementwise_source(root_shape, leaves, nodes, out_dtype):
-    """One thread per VECTOR consecutive elements in each of
+def elementwise_body(root_shape, leaves, nodes, out_dtype):
+    """(body, parameters, workgroups) of an elementwise group, the body for
+    workgroup `block`. One thread per VECTOR consecutive elements in each of
     ELEMENTS_PER_THREAD groups (a wave's group is 256 consecutive elements).
     A group whose operands all sit at 4-element alignment reads leaves that
     equal the root or repeat along leading axes (a bias) and writes the
@@ -251,12 +259,10 @@ def elementwise_source(root_shape, leaves, nodes, out_dtype):
         _, element_lines, element_result = _body(root_shape, leaves, nodes, leaf_value=leaf_value, suffix=suffix)
         per_element.append("{\n          " + "\n          ".join(element_lines) + f"\n          r[{e}] = {element_result};\n        }}")
     vector_body = "\n        ".join(per_element)
-    source = f"""{_PRELUDE}
-extern "C" __global__ __launch_bounds__({BLOCK}) void pacho_elementwise({", ".join(params)}) {{
-  const bool aligned = {aligned};
+    body = f"""  const bool aligned = {aligned};
 #pragma unroll
   for (int u = 0; u < {ELEMENTS_PER_THREAD}; ++u) {{
-    const {idx} i0 = (({idx})(blockIdx.x * {ELEMENTS_PER_THREAD}U + u) * {BLOCK}U + threadIdx.x) * {VECTOR}U;
+    const {idx} i0 = (({idx})(block * {ELEMENTS_PER_THREAD}U + u) * {BLOCK}U + threadIdx.x) * {VECTOR}U;
     if (aligned && i0 + {VECTOR}{suffix} <= {count}{suffix}) {{
         {loads}
         {t_out} r[{VECTOR}];
@@ -272,10 +278,19 @@ extern "C" __global__ __launch_bounds__({BLOCK}) void pacho_elementwise({", ".jo
         }}
       }}
     }}
-  }}
+  }}"""
+    return body, params, max(1, -(-count // span))
+
+
+def elementwise_source(root_shape, leaves, nodes, out_dtype):
+    """The kernel of an elementwise group and its workgroups."""
+    body, params, grid = elementwise_body(root_shape, leaves, nodes, out_dtype)
+    source = f"""{_PRELUDE}
+extern "C" __global__ __launch_bounds__({BLOCK}) void pacho_elementwise({", ".join(params)}) {{
+  const unsigned block = blockIdx.x;
+{body}
 }}
 """
-    grid = max(1, -(-count // span))
     return source, grid
 
 
@@ -365,6 +380,18 @@ class HIPLowering:
             and node.dtype.itemsize == 4
             and node.attrs.get("operation") in ("min", "max")
         )
+
+    def arrange(self, steps, outputs):
+        """The launches that compute a plan's steps (_hip_launches.py)."""
+        from ._hip_launches import arrange  # it builds on this module's sources
+
+        return arrange(self, steps, outputs)
+
+    def run_launch(self, nodes, payload, operands):
+        """Storage of every node of one Launch, in order."""
+        outs = [self.backend.empty(node.shape, node.dtype) for node in nodes]
+        self.backend._launch(payload.source, payload.name, payload.grid, operands, outs)
+        return outs
 
     def prepare_fused(self, node, group, leaves):
         specs, nodes = _graph(group, leaves)
