@@ -125,11 +125,11 @@ namespace {
 //   70 / 54, 1200 x 1200 x 2000 (2.9e9) 64 / 64; else 1000 x 3000 x 333 35 / 39,
 //   2500 x 2500 x 100 23 / 35. Products of the narrow kernel's extents stay
 //   there (1024^3 21 / 24, 8 x 512^3 21 / 30).
-//   fp64: 560 x 453 x 688 56 / 17, 1024^3 60 / 42, 2048 x 2048 x 256 65 / 57,
-//   8192 x 128 x 8192 575 / 291; large products 1200 x 1200 x 2000 125 / 133,
-//   2048^3 277 / 299; their kernel for any K (no multiple of 16) 1500^3
-//   168 / 142, 2672 x 2528 x 675 about even; few slices in many tiles 3025 x 2024
-//   x 75 33 / 55.
+//   fp64: 560 x 453 x 688 56 / 17, 1024^3 60 / 44, 128 x 8192 x 8192 577 / 303;
+//   whole staged tiles on half of the chip 2048 x 2048 x 256 62 / 66; large
+//   products 1200 x 1200 x 2000 125 / 133, 2048^3 277 / 299; the staged kernel
+//   for any K (no multiple of 16) 1500^3 166 / 130, 2000 x 600 x 3000 178 / 134;
+//   few slices in many tiles 3025 x 2024 x 75 33 / 55.
 bool direct_serves(int64_t cus, int dtype, int64_t m, int64_t n, int64_t k, int64_t batch) {
   const double work = double(m) * double(n) * double(k) * double(batch);
   const int64_t slices = hp::ceil_div(k, 16);
@@ -139,6 +139,7 @@ bool direct_serves(int64_t cus, int dtype, int64_t m, int64_t n, int64_t k, int6
   };
   if (dtype == HP_F64) {
     if (slices <= 8 && tiles64 > 2.0 * cus) return false;
+    if (k % 16 == 0 && m % 256 == 0 && n % 128 == 0 && double(m / 256) * double(n / 128) * batch * 2 >= cus) return false;
     return fill(256, 128) < 0.6 || work <= 2.4e9 || (k % 16 != 0 && slices >= 64 && work <= 8e9);
   }
   const bool narrow = m % 64 == 0 && n % 64 == 0 && k % 16 == 0 && tiles64 >= cus && tiles64 <= 4.0 * cus &&
@@ -173,6 +174,7 @@ hpgemm::DirectPlan hpgemm::direct_plan(int compute_units, int dtype, int64_t m, 
   const int64_t slices = hp::ceil_div(k, 16);
   const double unit = dtype == HP_F32 ? 0.053 : 0.107;  // us: one block over one slice
   for (const Candidate& c : kCandidates) {
+    if (c.fi * c.fj == 16 && dtype == HP_F64) continue;  // does not fit the registers
     // Tiles move inside the operands, which only one-block extents may undercut.
     if ((c.fi > 1 && m < 16 * c.fi) || (c.fj > 1 && n < 16 * c.fj)) continue;
     DirectPlan p;

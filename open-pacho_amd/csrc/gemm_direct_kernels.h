@@ -10,6 +10,16 @@ using hpgemm::BatchDesc;
 using hpgemm::DirectPlan;
 
 constexpr int kWaves = 4;  // per tile, each taking every fourth slice
+// Slices after which a wave's accumulators join its sums (DEPTH where that is
+// more): the chain of a sum is 4 MFMAs per slice of a run, then the runs of a
+// wave, so that its error stays below that of the staged kernels' cut tiles
+// (160 shapes, K up to 8192: 0.65 of theirs in the mean in fp32, 0.69 in fp64;
+// with one chain per wave it was up to 2.1 times theirs). Runs of 4 cost 3% of
+// the MFMA time; the 64 x 64 tile, whose registers are full, takes 8.
+template <int FI, int FJ>
+constexpr int run_slices() {
+  return FI * FJ == 16 ? 8 : 4;
+}
 constexpr int kGroupM = 4;  // tile rows per group: neighbours share operand panels in an XCD's L2
 
 template <typename T, int N>
@@ -142,11 +152,20 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? 2 : 1) void direct_ke
   oa.init(A + a_off, m0, M, t.lda, lane);
   ob.init(B + b_off, n0, N, t.ldb, lane);
 
-  Acc acc[FI][FJ];
+  Acc acc[FI][FJ], sums[FI][FJ];
 #pragma unroll
   for (int i = 0; i < FI; ++i)
 #pragma unroll
-    for (int j = 0; j < FJ; ++j) acc[i][j] = Acc{T(0), T(0), T(0), T(0)};
+    for (int j = 0; j < FJ; ++j) acc[i][j] = sums[i][j] = Acc{T(0), T(0), T(0), T(0)};
+  auto flush = [&] {
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+      for (int j = 0; j < FJ; ++j) {
+        sums[i][j] += acc[i][j];
+        acc[i][j] = Acc{T(0), T(0), T(0), T(0)};
+      }
+  };
 
   // This wave's slices: begin + wave, + kWaves, ...
   const int64_t begin = split * t.per_split;
@@ -171,11 +190,16 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? 2 : 1) void direct_ke
   for (int d = 0; d < DEPTH; ++d)
     if (d < count) load(d, a[d], b[d]);
   int64_t s = 0;
+  int run = 0;
   for (; s + 2 * DEPTH <= count; s += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
       fold(a[d], b[d]);
       load(s + DEPTH + d, a[d], b[d]);
+    }
+    if (++run == (run_slices<FI, FJ>() + DEPTH - 1) / DEPTH) {
+      flush();
+      run = 0;
     }
   }
   for (; s < count; s += DEPTH) {
@@ -184,6 +208,7 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? 2 : 1) void direct_ke
       if (s + d < count) fold(a[d], b[d]);
       if (s + DEPTH + d < count) load(s + DEPTH + d, a[d], b[d]);
     }
+    if constexpr (sizeof(T) == 4 && FI * FJ < 16) flush();
   }
 
   if (whole < end && (whole - begin) % kWaves == wave) {
@@ -192,6 +217,7 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? 2 : 1) void direct_ke
     ob.load_end(whole * 16, left, b[0]);
     fold(a[0], b[0]);
   }
+  flush();
 
   // Rows 16 at a time (those of accumulator blocks i): the waves' tiles meet in
   // LDS, are added in wave order and stored four columns per thread.
@@ -203,7 +229,7 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? 2 : 1) void direct_ke
 #pragma unroll
     for (int j = 0; j < FJ; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) stage[wave][Mfma<T>::row(lane, r) * kPitch + OB::row(j, lane & 15)] = acc[i][j][r];
+      for (int r = 0; r < 4; ++r) stage[wave][Mfma<T>::row(lane, r) * kPitch + OB::row(j, lane & 15)] = sums[i][j][r];
     __syncthreads();
     if (threadIdx.x < kThreads) {
       const int x = threadIdx.x / (4 * FJ), y = threadIdx.x % (4 * FJ) * 4;
@@ -280,8 +306,10 @@ void run_direct(hp_ctx* ctx, const DirectPlan& plan, bool ta, bool tb, const voi
   T* c = static_cast<T*>(c_);
   constexpr int kDeep = sizeof(T) == 4 ? 3 : 2;
   const int shape = plan.fi * 10 + plan.fj;
-  if (shape == 44) launch<T, 4, 4, kDeep>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
-  else if (shape == 42) launch<T, 4, 2, kDeep>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
+  if constexpr (sizeof(T) == 4) {  // in fp64 its accumulators, sums and fragments exceed the registers
+    if (shape == 44) return launch<T, 4, 4, 2>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
+  }
+  if (shape == 42) launch<T, 4, 2, kDeep>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
   else if (shape == 24) launch<T, 2, 4, kDeep>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
   else if (shape == 22) launch<T, 2, 2, 4>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
   else if (shape == 41) launch<T, 4, 1, 4>(ctx, plan, ta, tb, a, b, c, m, n, k, bd, batch);
