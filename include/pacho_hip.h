@@ -262,6 +262,12 @@ int hp_rtc_compile(hp_ctx* ctx, const char* source, const char* name, hp_kernel*
 int hp_rtc_launch(hp_ctx* ctx, hp_kernel* kernel, int64_t grid, int block, int shared_bytes,
                   void** args);
 
+/* hp_rtc_launch with the argument values themselves, laid out as the kernel's
+ * parameters are in memory: in order, each at its natural alignment, `bytes`
+ * (<= 4096) in all. The bytes are read before the call returns.
+ * Replaces: _cuda.py:359-374 (_run / cuLaunchKernel). */
+int hp_rtc_launch_packed(hp_ctx* ctx, hp_kernel* kernel, int64_t grid, int block, const void* args, int64_t bytes);
+
 /* Unload a compiled module. */
 int hp_rtc_release(hp_ctx* ctx, hp_kernel* kernel);
 

@@ -368,6 +368,22 @@ int hp_rtc_launch(hp_ctx* ctx, hp_kernel* kernel, int64_t grid, int block, int s
   });
 }
 
+int hp_rtc_launch_packed(hp_ctx* ctx, hp_kernel* kernel, int64_t grid, int block, const void* args, int64_t bytes) {
+  return guarded([&] {
+    hp::enter(ctx);
+    require(kernel != nullptr && kernel->function != nullptr, "null kernel");
+    require(grid >= 0 && grid <= hp::kMaxGrid, "grid out of range");
+    require(block > 0 && block <= 1024, "block out of range");
+    require(bytes >= 0 && bytes <= 4096 && (args != nullptr || bytes == 0), "argument bytes out of range");
+    if (grid == 0) return;
+    size_t size = static_cast<size_t>(bytes);
+    void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, const_cast<void*>(args), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
+                     HIP_LAUNCH_PARAM_END};
+    HP_CHECK(hipModuleLaunchKernel(kernel->function, static_cast<unsigned>(grid), 1, 1,
+                                   static_cast<unsigned>(block), 1, 1, 0, ctx->stream, nullptr, extra));
+  });
+}
+
 int hp_rtc_release(hp_ctx* ctx, hp_kernel* kernel) {
   return guarded([&] {
     require(ctx != nullptr, "null context");

@@ -352,10 +352,6 @@ class ExecutionPlan:
         # into (the steps stay what the plan is explained by).
         arrange = getattr(self.lowering, "arrange", None)
         self._launches = self.steps if arrange is None else arrange(self.steps, outputs)
-        # Reads of each value by later launches and by the result: a value is
-        # released when the count reaches zero.
-        self._reads = Counter(id(arg) for step in self._launches for arg in step.args)
-        self._reads.update(id(o) for o in outputs)
         self._executors = {
             "fused": self._run_fused,
             "map_reduce": self._run_map_reduce,
@@ -371,6 +367,59 @@ class ExecutionPlan:
             "reshape": lambda node, payload, operands: operands[0]._data,
             "full": lambda node, payload, operands: backend.full(node.shape, node.attrs["value"], node.dtype),
         }
+        self._assemble()
+
+    def _assemble(self):
+        """The launches as a program over numbered values: where each input and
+        scalar goes, then per launch what it runs, the values it reads, the
+        results it leaves (number, shape, dtype) and the values that nothing
+        reads after it."""
+        number = {}
+
+        def slot(node):
+            return number.setdefault(id(node), len(number))
+
+        sources = {}
+        for step in self._launches:
+            for node in (*step.args, *self._stored(step)):
+                slot(node)
+                if node.op in ("input", "scalar"):
+                    sources[id(node)] = node
+        for node in self.outputs:
+            slot(node)
+            if node.op in ("input", "scalar"):
+                sources[id(node)] = node
+        last = {id(arg): i for i, step in enumerate(self._launches) for arg in step.args}
+        kept = {id(node) for node in self.outputs}
+        self._inputs = [(slot(n), n.value.index) for n in sources.values() if n.op == "input"]
+        self._scalars = [(slot(n), n) for n in sources.values() if n.op == "scalar"]
+        self._program = []
+        for i, step in enumerate(self._launches):
+            results = [(slot(n), tuple(n.shape), np.dtype(n.dtype)) for n in self._stored(step)]
+            released = {slot(arg) for arg in step.args if last[id(arg)] == i and id(arg) not in kept}
+            run = self._runner(step)
+            self._program.append((run, [slot(arg) for arg in step.args], results, sorted(released)))
+        self._results = [slot(node) for node in self.outputs]
+        self._slots = len(number)
+
+    @staticmethod
+    def _stored(step):
+        return (step.node,) if isinstance(step, Step) else step.nodes
+
+    def _runner(self, step):
+        """A launch as a function of its operands' values, giving the storage of
+        its result, or the list of its results' storages."""
+        if not isinstance(step, Step):
+            return lambda operands: self.lowering.run_launch(step.nodes, step.payload, operands)
+        node, kind, args, payload = step
+        if kind in ELEMENTWISE:
+            return lambda operands: self._run_elementwise(node, kind, operands)
+        executor = self._executors.get(kind)
+        if executor is None:
+            raise NotImplementedError(f"No execution rule for {kind}")
+        if kind in ("fused", "map_reduce"):
+            return lambda operands: executor(node, payload, args, operands)
+        return lambda operands: executor(node, payload, [self._materialized(v) for v in operands])
 
     def execute(self, bindings):
         if self._execution_scope is None:
@@ -378,15 +427,11 @@ class ExecutionPlan:
         with self._execution_scope():
             return self._run(bindings)
 
-    def _leaf(self, node, bindings):
-        if node.op == "input":
-            return bindings[node.value.index]
-        if node.op == "scalar":
-            value = node.value
-            if isinstance(value, ScalarExpression):
-                return HostScalar(value.evaluate(bindings), node.dtype)
-            return value
-        raise RuntimeError(f"Missing plan dependency {node.op}")
+    def _scalar(self, node, bindings):
+        value = node.value
+        if isinstance(value, ScalarExpression):
+            return HostScalar(value.evaluate(bindings), node.dtype)
+        return value
 
     def _materialized(self, value):
         """A host scalar operand as a 0-d array (primitive steps take arrays)."""
@@ -395,39 +440,23 @@ class ExecutionPlan:
         return value
 
     def _run(self, bindings):
-        values, reads = {}, self._reads.copy()
-
-        def value_of(node):
-            if id(node) not in values:
-                values[id(node)] = self._leaf(node, bindings)
-            return values[id(node)]
-
-        def release(args):
-            for arg in args:
-                reads[id(arg)] -= 1
-                if not reads[id(arg)]:
-                    values.pop(id(arg), None)
-
-        for step in self._launches:
-            operands = [value_of(a) for a in step.args]
-            if not isinstance(step, Step):  # several values of one launch
-                for node, data in zip(step.nodes, self.lowering.run_launch(step.nodes, step.payload, operands)):
-                    values[id(node)] = ndarray._wrap(data, node.shape, node.dtype, self.backend)
-                release(step.args)
-                continue
-            node, kind, args, payload = step
-            if kind in ELEMENTWISE:
-                data = self._run_elementwise(node, kind, operands)
-            elif kind in ("fused", "map_reduce"):
-                data = self._executors[kind](node, payload, args, operands)
-            else:
-                executor = self._executors.get(kind)
-                if executor is None:
-                    raise NotImplementedError(f"No execution rule for {kind}")
-                data = executor(node, payload, [self._materialized(v) for v in operands])
-            values[id(node)] = ndarray._wrap(data, node.shape, node.dtype, self.backend)
-            release(args)
-        results = tuple(self._materialized(value_of(o)) for o in self.outputs)
+        values, backend = [None] * self._slots, self.backend
+        for slot, index in self._inputs:
+            values[slot] = bindings[index]
+        for slot, node in self._scalars:
+            values[slot] = self._scalar(node, bindings)
+        for run, reads, results, released in self._program:
+            data = run([values[slot] for slot in reads])
+            if len(results) == 1 and type(data) is not list:
+                data = (data,)
+            for storage, (slot, shape, dtype) in zip(data, results):
+                # ndarray._wrap without its checks: a plan's backend is not a
+                # trace, and shape and dtype are normalised.
+                values[slot] = array = object.__new__(ndarray)
+                array._data, array._shape, array._dtype, array._backend = storage, shape, dtype, backend
+            for slot in released:
+                values[slot] = None
+        results = tuple([self._materialized(values[slot]) for slot in self._results])
         return results if self.multiple else results[0]
 
     def _run_fused(self, node, payload, args, operands):
@@ -500,6 +529,22 @@ def _argument_spec(name, value, static):
     raise TypeError(f"Unsupported dynamic argument {name!r}; use static_argnames for metadata")
 
 
+def _quick_key(args):
+    """What the specs of a positional call follow from, where its arguments are
+    plain arrays and Python numbers: a key that costs less to build than the
+    specs. None for anything else."""
+    key = []
+    for value in args:
+        kind = type(value)
+        if kind is ndarray:
+            key.append((value._shape, value._dtype, value._backend))
+        elif kind is float or kind is bool or (kind is int and -(2**63) <= value < 2**63):
+            key.append(kind)
+        else:
+            return None
+    return tuple(key)
+
+
 class CompiledFunction:
     def __init__(self, function, static_argnames=(), cache_size=32, *, padding=False):
         self._padding = validate_padding(padding)
@@ -515,6 +560,8 @@ class CompiledFunction:
         self._positional = _all_positional(signature)
         self.max_size = cache_size
         self._plans = OrderedDict()
+        self._quick = {}  # _quick_key of a positional call -> its key in _plans
+        self._quick_names = len(self._names) if self._positional and not self.static_argnames else -1
         self._lock = RLock()
         self._hits = self._misses = 0
         update_wrapper(self, function)
@@ -530,6 +577,26 @@ class CompiledFunction:
         )
 
     def _plan(self, args, kwargs):
+        quick = None
+        if not kwargs and len(args) == self._quick_names:
+            quick = _quick_key(args)
+            if quick is not None:
+                with self._lock:
+                    key = self._quick.get(quick)
+                    plan = None if key is None else self._plans.get(key)
+                    if plan is not None:
+                        self._hits += 1
+                        self._plans.move_to_end(key)
+                        return plan, args
+        plan, bindings = self._find_plan(args, kwargs)
+        if quick is not None:
+            with self._lock:
+                if len(self._quick) >= 4 * self.max_size:
+                    self._quick.clear()
+                self._quick[quick] = self._specs(bindings)
+        return plan, bindings
+
+    def _find_plan(self, args, kwargs):
         bindings = _bindings(self.python_function, self._signature, self._positional, args, kwargs)
         key = self._specs(bindings)
         with self._lock:
@@ -549,7 +616,9 @@ class CompiledFunction:
 
     def __call__(self, *args, **kwargs):
         # Plain NumPy inputs run the original Python function unchanged.
-        if not any(isinstance(v, ndarray) for v in (*args, *kwargs.values())):
+        if not (args and type(args[0]) is ndarray) and not any(
+            isinstance(v, ndarray) for v in (*args, *kwargs.values())
+        ):
             return self.python_function(*args, **kwargs)
         plan, bindings = self._plan(args, kwargs)
         return plan.execute(bindings)
@@ -569,6 +638,7 @@ class CompiledFunction:
     def clear_cache(self):
         with self._lock:
             self._plans.clear()
+            self._quick.clear()
             self._hits = self._misses = 0
 
 

@@ -22,6 +22,7 @@ failing call raises.
 import ctypes
 from collections import OrderedDict
 from math import prod
+from struct import Struct
 from threading import RLock
 import weakref
 
@@ -39,14 +40,21 @@ _KERNEL_CACHE = 256
 # interchangeable; at most _SMALL_KEPT of them wait on the host for reuse.
 _SMALL_BLOCK = 512
 _SMALL_KEPT = 64
-_C_SCALARS = {
-    np.dtype("bool"): ctypes.c_uint8,
-    np.dtype("int32"): ctypes.c_int32,
-    np.dtype("int64"): ctypes.c_int64,
-    np.dtype("uint32"): ctypes.c_uint32,
-    np.dtype("uint64"): ctypes.c_uint64,
-    np.dtype("float32"): ctypes.c_float,
-    np.dtype("float64"): ctypes.c_double,
+# Blocks of the pool's power-of-two classes up to _KEPT_BLOCK wait on the host
+# too, at most _KEPT of each class (32 MiB in all), while the pool's limit is
+# far above that: a short operation's cost is its calls, and this saves two.
+_KEPT_BLOCK = 1 << 20
+_KEPT = 16
+_KEPT_POOL_LIMIT = 1 << 30
+# struct codes of scalar kernel arguments (native size and alignment).
+_SCALAR_CODES = {
+    np.dtype("bool"): "B",
+    np.dtype("int32"): "i",
+    np.dtype("int64"): "q",
+    np.dtype("uint32"): "I",
+    np.dtype("uint64"): "Q",
+    np.dtype("float32"): "f",
+    np.dtype("float64"): "d",
 }
 
 
@@ -157,7 +165,8 @@ class HIPBackend:
         self._leases = []
         self._lease_prune_at = 1024
         self._small = []  # returned blocks of <= _SMALL_BLOCK bytes, still live in the library
-        self._kernels = OrderedDict()
+        self._kept = {}  # size class -> returned blocks of that class (<= _KEPT_BLOCK), likewise
+        self._kernels = OrderedDict()  # source -> (kernel, packer of its arguments)
         self._ctx = None
         self._closed = False
         identifier = "0" if device is None else str(device)
@@ -175,7 +184,9 @@ class HIPBackend:
         self._ctx = ctx
         self._pool_limit = self.device_info.memory_bytes // 4  # hp_init's default
         # Bound once: the calls of the shortest operations are their cost.
+        self._alloc = self._lib.hp_alloc
         self._free = self._lib.hp_free
+        self._launch_packed = self._lib.hp_rtc_launch_packed
         self._dot = self._lib.hp_dot
         self._dot_new = self._lib.hp_dot_new
 
@@ -185,7 +196,8 @@ class HIPBackend:
         if self._closed:
             raise RuntimeError("hip backend is closed")
         status = getattr(self._lib, name)(self._ctx, *args)
-        lib_.check(self._lib, status, name)
+        if status:
+            lib_.check(self._lib, status, name)
 
     def _active(self):
         return self._guard
@@ -206,42 +218,60 @@ class HIPBackend:
         with self._lock:
             if self._closed:
                 return
-            if capacity <= _SMALL_BLOCK and len(self._small) < _SMALL_KEPT:
-                self._small.append(ptr)
-            else:
-                self._free(self._ctx, ptr)
+            if capacity <= _SMALL_BLOCK:
+                if len(self._small) < _SMALL_KEPT:
+                    self._small.append(ptr)
+                    return
+            elif capacity <= _KEPT_BLOCK and self._pool_limit >= _KEPT_POOL_LIMIT:
+                kept = self._kept.setdefault((capacity - 1).bit_length(), [])
+                if len(kept) < _KEPT:
+                    kept.append(ptr)
+                    return
+            self._free(self._ctx, ptr)
 
     def _return_small(self):
-        """Hand the host-side small blocks back to the library pool (called
-        with the backend lock held)."""
-        small, self._small = self._small, []
-        for ptr in small:
+        """Hand the blocks that wait on the host back to the library pool
+        (called with the backend lock held)."""
+        waiting = self._small + [ptr for kept in self._kept.values() for ptr in kept]
+        self._small, self._kept = [], {}
+        for ptr in waiting:
             lib_.check(self._lib, self._free(self._ctx, ptr), "hp_free")
 
     def _launch(self, source, name, grid, operands, out):
         """Compile (cached) and launch an RTC kernel over operands + out (one
         storage or a list of them)."""
-        with self._active():
-            kernel = self._kernels.get(source)
-            if kernel is None:
-                handle = ctypes.c_void_p()
-                self._call("hp_rtc_compile", source.encode(), name.encode(), ctypes.byref(handle))
-                if len(self._kernels) >= _KERNEL_CACHE:
-                    _, old = self._kernels.popitem(last=False)
-                    self._lib.hp_rtc_release(self._ctx, old)
-                kernel = self._kernels[source] = handle
+        with self._guard:
+            found = self._kernels.get(source)
+            if found is None:
+                found = self._compile(source, name, operands, out)
             else:
                 self._kernels.move_to_end(source)
-            values = []
-            for operand in operands:
-                if getattr(operand, "_host_scalar", False):
-                    values.append(_C_SCALARS[operand.dtype](operand._data.item()))
-                else:
-                    values.append(ctypes.c_void_p(operand._data.ptr))
-            for storage in out if isinstance(out, list) else (out,):
-                values.append(ctypes.c_void_p(storage.ptr))
-            pointers = (ctypes.c_void_p * len(values))(*(ctypes.addressof(v) for v in values))
-            self._call("hp_rtc_launch", kernel, grid, BLOCK, 0, pointers)
+            kernel, packer = found
+            values = [
+                operand._data.item() if getattr(operand, "_host_scalar", False) else operand._data.ptr
+                for operand in operands
+            ]
+            if type(out) is list:
+                values += [storage.ptr for storage in out]
+            else:
+                values.append(out.ptr)
+            status = self._launch_packed(self._ctx, kernel, grid, BLOCK, packer.pack(*values), packer.size)
+            if status:
+                lib_.check(self._lib, status, "hp_rtc_launch_packed")
+
+    def _compile(self, source, name, operands, out):
+        """Compile a source and keep it with the layout of its arguments, which
+        the source's parameters fix: operands (scalars by value, arrays as
+        pointers), then the outputs."""
+        handle = ctypes.c_void_p()
+        self._call("hp_rtc_compile", source.encode(), name.encode(), ctypes.byref(handle))
+        if len(self._kernels) >= _KERNEL_CACHE:
+            _, (old, _) = self._kernels.popitem(last=False)
+            self._lib.hp_rtc_release(self._ctx, old)
+        codes = [_SCALAR_CODES[v.dtype] if getattr(v, "_host_scalar", False) else "Q" for v in operands]
+        outputs = len(out) if type(out) is list else 1
+        self._kernels[source] = found = handle, Struct("@" + "".join(codes) + "Q" * outputs)
+        return found
 
     # ---- protocol: dtypes, storage, transfers --------------------------------------
 
@@ -259,11 +289,18 @@ class HIPBackend:
         if count > _MAX_ELEMENTS:
             raise ValueError("Array exceeds GPU indexing limits")
         capacity = max(1, count * dtype.itemsize)
-        with self._active():
-            if capacity <= _SMALL_BLOCK and self._small:
-                return _Allocation(self, self._small.pop(), capacity)
+        with self._guard:
+            if capacity <= _SMALL_BLOCK:
+                if self._small:
+                    return _Allocation(self, self._small.pop(), capacity)
+            elif capacity <= _KEPT_BLOCK:
+                kept = self._kept.get((capacity - 1).bit_length())
+                if kept:
+                    return _Allocation(self, kept.pop(), capacity)
             ptr = ctypes.c_void_p()
-            self._call("hp_alloc", capacity, ctypes.byref(ptr))
+            status = self._alloc(self._ctx, capacity, ptr)
+            if status:
+                lib_.check(self._lib, status, "hp_alloc")
             return _Allocation(self, ptr.value, capacity)
 
     def full(self, shape, value, dtype):
@@ -274,7 +311,7 @@ class HIPBackend:
             bits = np.asarray(value, dtype=dtype).tobytes().ljust(8, b"\0")
             pattern = int.from_bytes(bits[:8], "little")
             with self._active():
-                self._call("hp_fill", ctypes.c_void_p(out.ptr), count, dtype.itemsize, pattern)
+                self._call("hp_fill", out.ptr, count, dtype.itemsize, pattern)
         return out
 
     def upload(self, host):
@@ -282,7 +319,7 @@ class HIPBackend:
         out = self.empty(host.shape, host.dtype)
         if host.size:
             with self._active():
-                self._call("hp_h2d", ctypes.c_void_p(out.ptr), ctypes.c_void_p(host.ctypes.data), host.nbytes)
+                self._call("hp_h2d", out.ptr, host.ctypes.data, host.nbytes)
         return out
 
     def download(self, a):
@@ -290,7 +327,7 @@ class HIPBackend:
         with self._active():
             if not a._data.ptr:
                 raise RuntimeError("array storage was released when its hip backend closed")
-            self._call("hp_d2h", ctypes.c_void_p(out.ctypes.data), ctypes.c_void_p(a._data.ptr), out.nbytes)
+            self._call("hp_d2h", out.ctypes.data, a._data.ptr, out.nbytes)
         return out
 
     def synchronize(self):
@@ -348,8 +385,8 @@ class HIPBackend:
             self._call(
                 "hp_gather",
                 a.dtype.itemsize,
-                ctypes.c_void_p(a._data.ptr),
-                ctypes.c_void_p(out.ptr),
+                a._data.ptr,
+                out.ptr,
                 offset,
                 len(dims),
                 lib_.int64_array(dims),
@@ -403,8 +440,8 @@ class HIPBackend:
                     "hp_reduce",
                     lib_.DTYPE_CODES[dtype],
                     lib_.REDUCTIONS[operation],
-                    ctypes.c_void_p(source._data.ptr),
-                    ctypes.c_void_p(out.ptr),
+                    source._data.ptr,
+                    out.ptr,
                     outer,
                     reduced,
                     inner,
@@ -486,7 +523,7 @@ class HIPBackend:
 
     @staticmethod
     def _ptrs(*arrays):
-        return [ctypes.c_void_p(x.ptr if hasattr(x, "ptr") else x._data.ptr) for x in arrays]
+        return [x.ptr if type(x) is _Allocation else x._data.ptr for x in arrays]
 
     @staticmethod
     def _batch_strides(batch, a_batch, a_matrix, b_batch, b_matrix):
@@ -549,8 +586,8 @@ class HIPBackend:
                 self._call(
                     "hp_pad_copy",
                     array.dtype.itemsize,
-                    ctypes.c_void_p(array._data.ptr),
-                    ctypes.c_void_p(out.ptr),
+                    array._data.ptr,
+                    out.ptr,
                     prod(shape[:-2]),
                     array.shape[-2],
                     array.shape[-1],
@@ -572,8 +609,8 @@ class HIPBackend:
             self._call(
                 "hp_norm",
                 lib_.DTYPE_CODES[dtype],
-                ctypes.c_void_p(source._data.ptr),
-                ctypes.c_void_p(out.ptr),
+                source._data.ptr,
+                out.ptr,
                 outer,
                 reduced,
                 inner,
@@ -598,7 +635,7 @@ class HIPBackend:
                 "hp_philox",
                 lib_.DTYPE_CODES[dtype],
                 lib_.DISTRIBUTIONS[distribution],
-                ctypes.c_void_p(out.ptr),
+                out.ptr,
                 count,
                 seed,
                 start,
@@ -622,8 +659,8 @@ class HIPBackend:
                 if lease is not None:
                     lease.ptr = 0
             self._leases = []
-            self._small = []  # still live in the library: hp_destroy frees them
-            for kernel in self._kernels.values():
+            self._small, self._kept = [], {}  # still live in the library: hp_destroy frees them
+            for kernel, _ in self._kernels.values():
                 self._lib.hp_rtc_release(self._ctx, kernel)
             self._kernels.clear()
             if self._ctx is not None:

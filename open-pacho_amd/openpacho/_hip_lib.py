@@ -66,6 +66,7 @@ PROTOTYPES = {
     "hp_philox_words": [_ptr, _ptr, _i64, _u64, _u64],
     "hp_rtc_compile": [_ptr, _cstr, _cstr, _pptr],
     "hp_rtc_launch": [_ptr, _ptr, _i64, _i32, _i32, _pptr],
+    "hp_rtc_launch_packed": [_ptr, _ptr, _i64, _i32, _cstr, _i64],
     "hp_rtc_release": [_ptr, _ptr],
     "hp_event_create": [_ptr, _pptr],
     "hp_event_record": [_ptr, _ptr],
