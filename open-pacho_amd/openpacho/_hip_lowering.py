@@ -177,6 +177,32 @@ def _rows_of_four(root_shape, leaf_shape):
     return leaf_shape[-1] == root_shape[-1]
 
 
+def _four_values(root_shape, leaf_shape, k, leaf_type, idx, suffix):
+    """Source that leaves in l{k} what four consecutive root elements from i0
+    read of a leaf that repeats along leading axes (a row of features) or is
+    constant along trailing ones (a value per row), rows of any length: one
+    division for the four, one access for a row's part inside itself. None for
+    other leaves."""
+    lead = len(root_shape) - len(leaf_shape)
+    padded = (1,) * lead + tuple(leaf_shape)
+    size = prod(padded)
+    first = next((d for d, extent in enumerate(padded) if extent != 1), len(padded))
+    declare = f"{leaf_type} l{k}[{VECTOR}];"
+    if size >= VECTOR and padded[first:] == tuple(root_shape[first:]):
+        return (
+            f"{declare} {{ const {idx} at = i0 % {size}{suffix}; if (at + {VECTOR}{suffix} <= {size}{suffix}) pacho_loadu<false>(x{k} + at, l{k}); "
+            f"else {{ _Pragma(\"unroll\") for (int e = 0; e < {VECTOR}; ++e) l{k}[e] = x{k}[at + e < {size}{suffix} ? at + e : at + e - {size}{suffix}]; }} }}"
+        )
+    last = max((d for d, extent in enumerate(padded) if extent != 1), default=-1)
+    inner = prod(root_shape[last + 1 :])
+    if inner >= VECTOR and last >= 0 and padded[: last + 1] == tuple(root_shape[: last + 1]):
+        return (
+            f"{declare} {{ const {idx} at = i0 / {inner}{suffix}, past = i0 % {inner}{suffix}; "
+            f"_Pragma(\"unroll\") for (int e = 0; e < {VECTOR}; ++e) l{k}[e] = x{k}[past + e < {inner}{suffix} ? at : at + 1]; }}"
+        )
+    return None
+
+
 class _Leaf:
     __slots__ = ("scalar", "dtype", "shape")
 
@@ -227,8 +253,11 @@ def elementwise_body(root_shape, leaves, nodes, out_dtype):
     ELEMENTS_PER_THREAD groups (a wave's group is 256 consecutive elements).
     A group whose operands all sit at 4-element alignment reads leaves that
     equal the root or repeat along leading axes (a bias) and writes the
-    output with one vector access each (16 bytes for 4-byte types); other
-    leaves, the tail and misaligned operands go element by element. Every
+    output with one vector access each (16 bytes for 4-byte types); leaves that
+    repeat or are constant along rows of any length take one division
+    (_four_values: the quotient of a centred 100003 x 1025 float32 array by a
+    row of deviations 227 -> 133 us); other leaves, the tail and misaligned
+    operands go element by element. Every
     element computes the same expression as in the element-by-element form,
     so the bits do not depend on the path."""
     count = prod(root_shape)
@@ -249,10 +278,16 @@ def elementwise_body(root_shape, leaves, nodes, out_dtype):
         f"({_broadcast_offset(root_shape, leaves[k].shape, 'i0', suffix)}), l{k});"
         for k in rows
     )
+    four = {
+        k: _four_values(tuple(root_shape), leaf.shape, k, ctype(leaf.dtype), idx, suffix)
+        for k, leaf in enumerate(leaves)
+        if not leaf.scalar and k not in rows
+    }
+    loads = "\n        ".join([loads, *filter(None, four.values())])
     per_element = []
     for e in range(VECTOR):
         def leaf_value(k, e=e):
-            if k in rows:
+            if k in rows or four[k]:
                 return f"l{k}[{e}]"
             return f"x{k}[{_broadcast_offset(root_shape, leaves[k].shape, f'(i0 + {e}{suffix})', suffix)}]"
 
