@@ -8,7 +8,7 @@ the elementwise sources (_hip_lowering.py); only the order of a sum depends on
 the kernel, and it is fixed for a shape, so results repeat bit for bit.
 """
 
-from math import prod
+from math import gcd, prod
 
 from . import _hip_lowering as source_
 
@@ -229,15 +229,16 @@ LEAST_ROWS = 16
 MOST_PARTIAL_BYTES = 8 << 20
 
 
-def _column_plan(outer, reduced, inner, width, acc_bytes):
+def _column_plan(outer, reduced, inner, width, acc_bytes, unit=1):
     """(groups of `width` columns a workgroup spans, column blocks, rows per
     step, rows per chunk, chunks). Of the ways to cut a row into equal blocks
-    of at least 16 groups (256 bytes of 4-byte columns), the one that leaves
-    the fewest threads without a column, the widest of equals."""
+    of at least 16 groups (256 bytes of 4-byte columns), a multiple of `unit`,
+    the one that leaves the fewest threads without a column, the widest of
+    equals."""
     groups = -(-inner // width)
     best, fewest = None, -(-groups // BLOCK)
     for blocks in range(fewest, min(max(fewest, groups // 16), fewest + 32) + 1):
-        across = -(-groups // blocks)
+        across = -(-(-(-groups // blocks)) // unit) * unit
         used = groups * (BLOCK // across) / (-(-groups // across) * BLOCK)
         if best is None or used > best[0] + 0.02:
             best = used, across
@@ -250,49 +251,79 @@ def _column_plan(outer, reduced, inner, width, acc_bytes):
     return across, blocks, step, rows, -(-reduced // rows)
 
 
+def _folded_rows(m, width):
+    """Rows that the column kernel takes as one long row, so that every long
+    row starts at the same place of a 128-byte line (of a 16-byte vector for
+    fewer rows), and whether it is the line; 1 where rows are whole vectors,
+    where a leaf varies along the rows, where too few long rows would be left
+    for each of their columns' own partial, or where one launch of single
+    columns does it without partials."""
+    if m.inner % width == 0 or m.reads("reduced"):
+        return 1, False
+    if _column_plan(m.outer, m.reduced, m.inner, 1, m.acc_dtype.itemsize)[4] == 1:
+        return 1, False
+    for period, least in ((8 * width, 64), (width, 16)):
+        rows = period // gcd(m.inner, period)
+        if m.reduced >= least * rows and m.outer * rows * m.inner * m.acc_dtype.itemsize <= MOST_PARTIAL_BYTES:
+            return rows, period > width
+    return 1, False
+
+
 def _columns(m):
     """A workgroup owns a block of columns and a chunk of rows; a thread reads
     `width` adjacent columns of every step-th row, eight rows (16 of one
-    column) in flight. Each batch folds on its own before it joins the
-    accumulator, so the chain of a sum is rows / 8 long; the rows of a step
+    column) in flight. Each batch folds on its own, in pairs, before it joins
+    the accumulator, so the chain of a sum is rows / 8 long; the rows of a step
     meet in LDS in a fixed tree. Leaves that vary along inner only are read
     once. Bound by HBM: where rows are whole vectors a thread takes 16 bytes
     with the nontemporal hint (100003 x 1024 float32: 67 us, 6.1 TB/s, against
-    78 us without the hint), else one column without it, since the lines at a
-    row's ends are shared (100003 x 1025: 89 us, 4.6 TB/s, against 122 us for
-    16 bytes at element alignment). Workgroups are renumbered so that an XCD
+    78 us without the hint). Other rows are folded (_folded_rows): 32 rows of
+    1025 float32 are one row of 32800 columns that starts on a line, whose
+    partials are 32 rows of the result's partials, and the last, cut long row
+    goes element by element: the sum of squares of 100003 x 1025 float32 88 us
+    by single columns, 73 with long rows that start on 16 bytes, 67 on lines.
+    Where that does not serve, a thread takes one column without the hint. Workgroups are renumbered so that an XCD
     (ids i % 8) owns neighbouring column blocks, which share lines. With a
     lane per row of one column and 64 lines per wave access, the mean square
     over axis 0 of 100003 x 1025 took 1062 us."""
     wide = max([m.acc_dtype.itemsize, *(leaf.dtype.itemsize for leaf in m.leaves if not leaf.scalar)]) == 8
     width, batch = 2 if wide else 4, 8
     stream = "true"
-    if m.inner % width:
+    folded, lines_whole = _folded_rows(m, width)
+    if folded == 1 and m.inner % width:
         width, batch, stream = 1, 16, "false"
-    across, blocks, step, rows, chunks = _column_plan(m.outer, m.reduced, m.inner, width, m.acc_dtype.itemsize)
+    inner, total = folded * m.inner, m.reduced * m.inner
+    reduced = -(-m.reduced // folded)
+    across, blocks, step, rows, chunks = _column_plan(
+        m.outer, reduced, inner, width, m.acc_dtype.itemsize, 8 if lines_whole else 1
+    )
     grid = m.outer * chunks * blocks
     lambdas, given = m.lambdas("full", "reduced", "outer", "inner", "one")
     constants = [f"const {t} s{k} = x{k}[{'o' if m.access[k] == 'outer' else '0'}];" for k, t in m.reads("outer", "one")]
     for k, t in m.reads("inner"):
-        constants.append(f"{t} c{k}[{width}]; pacho_loadu<false>(x{k} + col, c{k});")
+        each = f"_Pragma(\"unroll\") for (int v = 0; v < {width}; ++v) c{k}[v] = x{k}[(col + v) % {m.inner}LL];"
+        constants.append(f"{t} c{k}[{width}]; " + (each if folded > 1 else f"pacho_loadu<false>(x{k} + col, c{k});"))
 
     def loads(j):
-        at = f"first + r * {m.inner}LL + {j * step * m.inner}LL"
+        at = f"first + r * {inner}LL + {j * step * inner}LL"
         lines = [f"{t} l{j}_{k}[{width}]; pacho_loadu<{stream}>(x{k} + ({at}), l{j}_{k});" for k, t in m.reads("full")]
         return lines + [f"const {t} l{j}_{k} = x{k}[r + {j * step}];" for k, t in m.reads("reduced")]
 
     def value(j, v):
         names = {"full": f"l{j}_%d[{v}]", "reduced": f"l{j}_%d", "inner": f"c%d[{v}]"}
         arguments = "".join(", " + names.get(m.access[k], "s%d") % k for k in given)
-        return f"mapped(first + r * {m.inner}LL + {j * step * m.inner + v}LL{arguments})"
+        return f"mapped(first + r * {inner}LL + {j * step * inner + v}LL{arguments})"
 
     def fold(count):
         lines = []
         for v in range(width):
-            lines += ["{", f"  {m.acc} some = {value(0, v)};"]
-            for j in range(1, count):
-                lines += ["  {", f"    const {m.acc} next = {value(j, v)};", f"    some = {m.combine('some', 'next')};", "  }"]
-            lines += [f"  acc[{v}] = {m.combine(f'acc[{v}]', 'some')};", "}"]
+            lines += ["{", *(f"  {m.acc} some{j} = {value(j, v)};" for j in range(count))]
+            apart = 1
+            while apart < count:
+                for j in range(0, count - apart, 2 * apart):
+                    lines.append(f"  some{j} = {m.combine(f'some{j}', f'some{j + apart}')};")
+                apart *= 2
+            lines += [f"  acc[{v}] = {m.combine(f'acc[{v}]', 'some0')};", "}"]
         return lines
 
     tree = f"""
@@ -318,40 +349,40 @@ def _columns(m):
   const long long o = id / {blocks * chunks}U;
   const int row = threadIdx.x / {across};
   const long long col = (block * {across}LL + threadIdx.x % {across}) * {width};
-  const bool active = row < {step} && block * {across} + threadIdx.x % {across} < {-(-m.inner // width)};
-  const long long first = o * {m.reduced * m.inner}LL + col;
+  const bool active = row < {step} && col < {inner}LL;
+  const long long first = o * {total}LL + col;
   const long long begin = chunk * {rows}LL;
-  const long long end = begin + {rows}LL < {m.reduced}LL ? begin + {rows}LL : {m.reduced}LL;
+  const long long end = begin + {rows}LL < {reduced}LL ? begin + {rows}LL : {reduced}LL;
+  // Rows that hold all of this thread's columns: all but the last of folded ones.
+  const long long full = ({total}LL - col - {width} + {inner}LL) / {inner}LL, whole = full < end ? full : end;
   {m.acc} acc[{width}];
 #pragma unroll
   for (int v = 0; v < {width}; ++v) acc[v] = {m.identity};
-  if (active && col + {width} <= {m.inner}LL) {{
+  if (active) {{
     {_lines(constants, 4)}
     long long r = begin + row;
-    for (; r + {(batch - 1) * step} < end; r += {batch * step}) {{
+    for (; r + {(batch - 1) * step} < whole; r += {batch * step}) {{
       {_lines([line for j in range(batch) for line in loads(j)], 6)}
       {FENCE}
       {_lines(fold(batch), 6)}
     }}
-    for (; r < end; r += {step}) {{
+    for (; r < whole; r += {step}) {{
       {_lines(loads(0), 6)}
       {_lines(fold(1), 6)}
     }}
-  }} else if (active) {{  // the last columns of an inner extent that is no multiple of {width}
-    for (long long r = begin + row; r < end; r += {step}) {{
+    if (r < end) {{
       for (int v = 0; v < {width}; ++v) {{
-        if (col + v < {m.inner}LL) {{
-          const {m.acc} value = element(first + r * {m.inner}LL + v);
+        if (r * {inner}LL + col + v < {total}LL) {{
+          const {m.acc} value = element(first + r * {inner}LL + v);
           acc[v] = {m.combine("acc[v]", "value")};
         }}
       }}
     }}
   }}{tree}
   if (active && row == 0) {{
-    for (int v = 0; v < {width}; ++v)
-      if (col + v < {m.inner}LL) out[(o * {chunks}LL + chunk) * {m.inner}LL + col + v] = acc[v];
+    for (int v = 0; v < {width}; ++v) out[(o * {chunks}LL + chunk) * {inner}LL + col + v] = acc[v];
   }}"""
-    return MapReduce(m.kernel(body), m.outer * m.inner, chunks, grid, (m.outer, chunks, m.inner))
+    return MapReduce(m.kernel(body), m.outer * m.inner, chunks * folded, grid, (m.outer, chunks * folded, m.inner))
 
 
 def _any(m):

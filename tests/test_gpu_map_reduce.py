@@ -51,6 +51,62 @@ def test_mapped_reductions_are_exact_on_small_integers(hip, shape, axes, index):
         np.testing.assert_array_equal(got, function(host * other - 2, axis=axes))
 
 
+# Rows folded into long ones: by lines and by vectors, with every kind of last
+# row, at the edges of the rule (64 long rows of lines, 16 of vectors), batched.
+FOLDED = [((rows, 5), (0,)) for rows in (64, 816, 817, 1024, 1027, 2047, 2048, 2049, 2079, 2080)]
+FOLDED += [((4 * 1024 + 3, 1025), (0,)), ((3001, 14), (0,)), ((40001, 6), (0,)), ((3, 2051, 7), (1,)), ((2, 30, 71, 9), (1, 2))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,axes", FOLDED)
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+def test_folded_rows_are_exact_on_small_integers(hip, shape, axes, dtype):
+    rng = np.random.default_rng(5)
+    host = rng.integers(-3, 4, shape).astype(dtype)
+    x = p.asarray(host, backend=hip)
+    for kind in _leaf_shapes(shape):
+        other = rng.integers(-3, 4, kind).astype(dtype)
+        sums, most = p.compile(lambda x, b: (np.sum(x * b - 2, axis=axes), np.max(x - b, axis=axes)))(
+            x, p.asarray(other, backend=hip)
+        )
+        np.testing.assert_array_equal(p.asnumpy(sums), np.sum(host * other - 2, axis=axes))
+        np.testing.assert_array_equal(p.asnumpy(most), np.max(host - other, axis=axes))
+
+
+def _touched(shape, axes, leaf, dtype):
+    """How often the column kernel's index arithmetic reads each element, and the partials it leaves."""
+    from openpacho._hip_map_reduce import _Mapped, _folded_rows
+
+    m = _Mapped(shape, axes, [_Leaf(False, dtype, shape), _Leaf(False, dtype, leaf)], [("add", [0, 1], (dtype,) * 2, dtype)], "sum", dtype)
+    width = 16 // dtype.itemsize
+    folded, lines = _folded_rows(m, width)
+    if folded == 1:
+        return folded, None
+    inner, total, reduced = folded * m.inner, m.reduced * m.inner, -(-m.reduced // folded)
+    across, blocks, step, rows, chunks = _column_plan(m.outer, reduced, inner, width, dtype.itemsize, 8 if lines else 1)
+    touched = np.zeros(total, int)
+    for col in range(0, inner, width):
+        for chunk in range(chunks):
+            end = min((chunk + 1) * rows, reduced)
+            whole = min((total - col - width + inner) // inner, end)
+            r = np.arange(chunk * rows, end)
+            for v in range(width):
+                at = r * inner + col + v
+                assert np.all(at[r < whole] < total) and np.sum(r >= whole) <= 1
+                touched[at[at < total]] += 1
+    assert across * step <= BLOCK and (blocks - 1) * across * width < inner <= blocks * across * width
+    return folded, touched
+
+
+@pytest.mark.parametrize("shape,axes", FOLDED)
+@pytest.mark.parametrize("dtype", ["f4", "f8"])
+def test_folded_rows_read_every_element_once(shape, axes, dtype):
+    folded, touched = _touched(shape, axes, shape[-1:], np.dtype(dtype))
+    if shape[0] >= 2048 and shape[-1] % 2:
+        assert folded > 1
+    assert touched is None or np.all(touched == 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,axis", [((37, 5000), 1), ((9000, 49), 1), ((3, 20000), 1), ((20000, 129), 0)])
 def test_mapped_sums_round_like_the_eager_sum_and_within_their_bound(hip, shape, axis):
