@@ -22,7 +22,7 @@ failing call raises.
 import ctypes
 from collections import OrderedDict
 from math import prod
-from struct import Struct
+from struct import Struct, calcsize
 from threading import RLock
 import weakref
 
@@ -46,6 +46,7 @@ _SMALL_KEPT = 64
 _KEPT_BLOCK = 1 << 20
 _KEPT = 16
 _KEPT_POOL_LIMIT = 1 << 30
+_PACKED_BYTES = 4096  # of arguments that hp_rtc_launch_packed takes
 # struct codes of scalar kernel arguments (native size and alignment).
 _SCALAR_CODES = {
     np.dtype("bool"): "B",
@@ -255,9 +256,23 @@ class HIPBackend:
                 values += [storage.ptr for storage in out]
             else:
                 values.append(out.ptr)
-            status = self._launch_packed(self._ctx, kernel, grid, BLOCK, packer.pack(*values), packer.size)
+            packed = packer.pack(*values)
+            if len(packed) > _PACKED_BYTES:
+                self._launch_pointers(kernel, grid, packer.format, packed)
+                return
+            status = self._launch_packed(self._ctx, kernel, grid, BLOCK, packed, packer.size)
             if status:
                 lib_.check(self._lib, status, "hp_rtc_launch_packed")
+
+    def _launch_pointers(self, kernel, grid, layout, packed):
+        """Launch with a pointer to each argument inside `packed` (of the struct
+        `layout`), as many arguments as there are."""
+        buffer = ctypes.create_string_buffer(packed, len(packed))
+        base = ctypes.addressof(buffer)
+        ends = [calcsize(layout[: i + 1]) for i in range(1, len(layout))]
+        starts = [end - calcsize("=" + code) for end, code in zip(ends, layout[1:])]
+        pointers = (ctypes.c_void_p * len(starts))(*(base + at for at in starts))
+        self._call("hp_rtc_launch", kernel, grid, BLOCK, 0, pointers)
 
     def _compile(self, source, name, operands, out):
         """Compile a source and keep it with the layout of its arguments, which

@@ -37,6 +37,7 @@ CHEAP = frozenset(
 )
 MOST_REPEATED = 4  # nodes of an inlined value
 MOST_MERGED = 8  # outputs of a merged launch
+MOST_ARGUMENTS = 256  # operands of its members together: far below what a packed launch takes
 SMALL = 1 << 16  # elements up to which a step may run later than the plan has it
 MOST_REGISTERS = 160  # 32-bit registers of row values per lane
 
@@ -412,7 +413,8 @@ def _merge(launches):
                 if len(members) == MOST_MERGED or any(id(arg) in stored for arg in later.args):
                     break
                 small = all(prod(s.node.shape) <= SMALL for s in members)
-                if _is_fused(later) and (small or last == i - 1):
+                operands = sum(len(s.args) for s in members) + len(later.args)
+                if _is_fused(later) and (small or last == i - 1) and operands <= MOST_ARGUMENTS:
                     members.append(later)
                     last = i
                 elif not small:

@@ -152,3 +152,23 @@ def test_scalars_rebind_and_dtypes_mix_in_regrouped_launches(hip, monkeypatch):
         for got, want in zip(compiled(x, scale), mixed(host, np.int32(scale))):
             np.testing.assert_array_equal(p.asnumpy(got), want)
     assert compiled.cache_info()["misses"] == 1
+
+
+@pytest.mark.parametrize("count", [40, 505, 520])
+def test_many_operands(hip, count):
+    # Several groups whose operands together pass what one launch packs, and one
+    # group around that limit (505 and 520 pointers, a flag and a number).
+    host = [np.full(70, i % 7, np.int32) for i in range(count)]
+    arrays = [p.asarray(v, backend=hip) for v in host]
+
+    def total(values):
+        return values[0] if len(values) == 1 else total(values[: len(values) // 2]) + total(values[len(values) // 2 :])
+
+    names = [f"a{i}" for i in range(count)]
+    scope = {"total": total}
+    result = "total(a) * flag + scale" if count > 100 else "tuple(total(a) * flag + scale + j for j in range(8))"
+    exec(f"def function(flag, {', '.join(names)}, scale):\n    a = [{', '.join(names)}]\n    return {result}", scope)
+    function = scope["function"]
+    got, want = p.compile(function)(True, *arrays, 3), function(True, *host, 3)
+    for g, w in zip(*(v if isinstance(v, tuple) else (v,) for v in (got, want))):
+        np.testing.assert_array_equal(p.asnumpy(g), w)
