@@ -232,11 +232,15 @@ class HIPBackend:
 
     def _return_small(self):
         """Hand the blocks that wait on the host back to the library pool
-        (called with the backend lock held)."""
-        waiting = self._small + [ptr for kept in self._kept.values() for ptr in kept]
-        self._small, self._kept = [], {}
-        for ptr in waiting:
-            lib_.check(self._lib, self._free(self._ctx, ptr), "hp_free")
+        (called with the backend lock held). A finaliser may return a block
+        between any two instructions here, so the lists are held by name
+        before they are replaced: it lands in the old list, which is still to
+        be walked, or in the new one."""
+        small, self._small = self._small, []
+        kept, self._kept = self._kept, {}
+        for waiting in (small, *kept.values()):
+            for ptr in waiting:
+                lib_.check(self._lib, self._free(self._ctx, ptr), "hp_free")
 
     def _launch(self, source, name, grid, operands, out):
         """Compile (cached) and launch an RTC kernel over operands + out (one

@@ -1,0 +1,114 @@
+"""Host side of HIPBackend without a device: its blocks and their lifetime on a
+stand-in library that hands out numbers as addresses and keeps account of them."""
+
+import ctypes
+import sys
+
+import numpy as np
+import pytest
+
+from openpacho import _hip, _hip_lib
+from openpacho.backends import DeviceInfo
+
+
+class Library:
+    """The entry points that storage uses. ``live`` holds the addresses given
+    out; ``after`` is called at the start of an entry point of that name."""
+
+    def __init__(self):
+        self.live, self.next, self.limit, self.after = set(), 1 << 20, None, {}
+
+    def _enter(self, name):
+        if name in self.after:
+            self.after[name]()
+
+    def hp_init(self, ordinal, out):
+        out._obj.value = 1
+        return 0
+
+    def hp_alloc(self, ctx, bytes, out):
+        self._enter("hp_alloc")
+        self.next += 1 << 20
+        out.value = self.next
+        self.live.add(self.next)
+        return 0
+
+    def hp_free(self, ctx, ptr):
+        self.live.remove(ptr)
+        return 0
+
+    def hp_set_pool_limit(self, ctx, value):
+        self._enter("hp_set_pool_limit")
+        self.limit = value
+        return 0
+
+    def hp_release_cached(self, ctx):
+        return 0
+
+    def hp_destroy(self, ctx):
+        return 0
+
+    def hp_last_error(self):
+        return b""
+
+    def __getattr__(self, name):  # bound by the backend, unused here
+        if name.startswith("hp_"):
+            return None
+        raise AttributeError(name)
+
+
+@pytest.fixture
+def backend(monkeypatch):
+    device = DeviceInfo("0", "stand-in", "AMD", "GPU", True, 256 << 30, "")
+    monkeypatch.setattr(_hip, "hip_devices", lambda: [device])
+    monkeypatch.setattr(_hip_lib, "load", Library)
+    made = _hip.HIPBackend()
+    yield made
+    made.close()
+
+
+def _waiting(backend):
+    return list(backend._small) + [ptr for kept in backend._kept.values() for ptr in kept]
+
+
+def _at_instruction(function, number, action):
+    """Call ``function``; before its ``number``-th instruction call ``action``.
+    False when the function has fewer instructions."""
+    code, left = function.__func__.__code__, [number]
+
+    def trace(frame, event, arg):
+        if frame.f_code is not code:
+            return None
+        frame.f_trace_opcodes = True
+        if event == "opcode":
+            left[0] -= 1
+            if left[0] == 0:
+                sys.settrace(None)
+                action()
+                sys.settrace(trace)
+        return trace
+
+    sys.settrace(trace)
+    try:
+        function()
+    finally:
+        sys.settrace(None)
+    return left[0] <= 0
+
+
+def test_a_block_dropped_while_the_waiting_ones_go_back_is_not_lost(backend):
+    # The garbage collector may run a finaliser between any two instructions:
+    # one drops a block of another class there, and every block is afterwards
+    # either back in the library or waiting.
+    number, reached = 0, True
+    while reached:
+        number += 1
+        blocks = [backend.empty((n,), np.bool_) for n in (3, 40, 5000, 70000)]
+        late = [backend.empty((n,), np.bool_) for n in (9, 300000)]
+        blocks.clear()
+        with backend._lock:
+            reached = _at_instruction(backend._return_small, number, late.clear)
+        late.clear()
+        assert set(_waiting(backend)) == backend._lib.live, f"before instruction {number}"
+        assert len(_waiting(backend)) == len(set(_waiting(backend)))
+    assert number > 10
