@@ -196,9 +196,20 @@ class HIPBackend:
     def _call(self, name, *args):
         if self._closed:
             raise RuntimeError("hip backend is closed")
-        status = getattr(self._lib, name)(self._ctx, *args)
+        function = getattr(self._lib, name)
+        status = function(self._ctx, *args)
         if status:
-            lib_.check(self._lib, status, name)
+            lib_.check(self._lib, self._again(status, function, *args), name)
+
+    def _again(self, status, function, *args):
+        """The status of a failed call, or of a second try where memory ran
+        out while blocks waited on the host: the library releases only blocks
+        that it knows to be free. A call writes its outputs alone, so it can be
+        repeated (called with the backend lock held)."""
+        if status == lib_.HP_E_OOM and (self._small or self._kept):
+            self._return_small()
+            status = function(self._ctx, *args)
+        return status
 
     def _active(self):
         return self._guard
@@ -319,7 +330,7 @@ class HIPBackend:
             ptr = ctypes.c_void_p()
             status = self._alloc(self._ctx, capacity, ptr)
             if status:
-                lib_.check(self._lib, status, "hp_alloc")
+                lib_.check(self._lib, self._again(status, self._alloc, capacity, ptr), "hp_alloc")
             return _Allocation(self, ptr.value, capacity)
 
     def full(self, shape, value, dtype):
@@ -513,15 +524,19 @@ class HIPBackend:
             small = self._small
             if small:
                 block = small.pop()
-                status = self._dot(self._ctx, lib_.DTYPE_CODES[dtype], a._data.ptr, b._data.ptr, block, a._shape[0])
+                arguments = lib_.DTYPE_CODES[dtype], a._data.ptr, b._data.ptr, block, a._shape[0]
+                status = self._dot(self._ctx, *arguments)
                 if status:
-                    small.append(block)
+                    status = self._again(status, self._dot, *arguments)
+                if status:
+                    self._small.append(block)
                     lib_.check(self._lib, status, "hp_dot")
                 return _Allocation(self, block, dtype.itemsize)
             ptr = ctypes.c_void_p()
-            status = self._dot_new(self._ctx, lib_.DTYPE_CODES[dtype], a._data.ptr, b._data.ptr, a._shape[0], ptr)
+            arguments = lib_.DTYPE_CODES[dtype], a._data.ptr, b._data.ptr, a._shape[0], ptr
+            status = self._dot_new(self._ctx, *arguments)
             if status:
-                lib_.check(self._lib, status, "hp_dot_new")
+                lib_.check(self._lib, self._again(status, self._dot_new, *arguments), "hp_dot_new")
             return _Allocation(self, ptr.value, dtype.itemsize)
 
     def _gemm(self, code, a, b, out, m, n, k, batch, a_batch, b_batch):

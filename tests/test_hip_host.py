@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from openpacho import _hip, _hip_lib
+from openpacho._array import ndarray
 from openpacho.backends import DeviceInfo
 
 
@@ -17,6 +18,7 @@ class Library:
 
     def __init__(self):
         self.live, self.next, self.limit, self.after = set(), 1 << 20, None, {}
+        self.most = None  # live blocks that memory has room for
 
     def _enter(self, name):
         if name in self.after:
@@ -28,10 +30,21 @@ class Library:
 
     def hp_alloc(self, ctx, bytes, out):
         self._enter("hp_alloc")
+        if self.most is not None and len(self.live) >= self.most:
+            return _hip_lib.HP_E_OOM
         self.next += 1 << 20
         out.value = self.next
         self.live.add(self.next)
         return 0
+
+    def hp_dot_new(self, ctx, code, a, b, n, out):
+        return self.hp_alloc(ctx, 8, out)
+
+    def hp_gemv(self, ctx, *args):
+        """Needs one block of its own while it runs."""
+        scratch = ctypes.c_void_p()
+        status = self.hp_alloc(ctx, 1, scratch)
+        return status or self.hp_free(ctx, scratch.value)
 
     def hp_free(self, ctx, ptr):
         self.live.remove(ptr)
@@ -112,3 +125,41 @@ def test_a_block_dropped_while_the_waiting_ones_go_back_is_not_lost(backend):
         assert set(_waiting(backend)) == backend._lib.live, f"before instruction {number}"
         assert len(_waiting(backend)) == len(set(_waiting(backend)))
     assert number > 10
+
+
+def _out_of_memory(backend, live):
+    """``live`` blocks in use, others waiting, and no memory for any more."""
+    used = [backend.empty((100000,), np.bool_) for _ in range(live)]
+    dropped = [backend.empty((n,), np.bool_) for n in (5000, 5000, 70000)]
+    dropped.clear()
+    backend._lib.most = len(backend._lib.live)
+    assert len(_waiting(backend)) == 3
+    return used
+
+
+def test_waiting_blocks_go_back_before_an_allocation_fails(backend):
+    used = _out_of_memory(backend, 2)
+    used.append(backend.empty((1 << 21,), np.bool_))  # no block of its class waits
+    assert not _waiting(backend) and len(backend._lib.live) == 3
+    backend._lib.most = 3
+    with pytest.raises(RuntimeError, match="hp_alloc"):
+        backend.empty((1 << 21,), np.bool_)
+
+
+def test_waiting_blocks_go_back_before_a_call_that_needs_memory_fails(backend):
+    used = _out_of_memory(backend, 1)
+    backend._call("hp_gemv")
+    assert not _waiting(backend) and backend._lib.live == {used[0].ptr}
+    backend._lib.most = 1
+    with pytest.raises(RuntimeError, match="hp_gemv"):
+        backend._call("hp_gemv")
+
+
+def test_waiting_blocks_go_back_before_a_dot_fails(backend):
+    used = _out_of_memory(backend, 1)
+    vector = ndarray._wrap(used[0], (10,), np.dtype("float32"), backend)
+    out = backend.vector_dot(vector, vector)
+    assert not _waiting(backend) and backend._lib.live == {used[0].ptr, out.ptr}
+    backend._lib.most = 2
+    with pytest.raises(RuntimeError, match="hp_dot_new"):
+        backend.vector_dot(vector, vector)
