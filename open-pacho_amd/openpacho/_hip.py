@@ -382,9 +382,14 @@ class HIPBackend:
         if value < 0:
             raise ValueError("pool limit must be non-negative")
         with self._active():
-            self._return_small()
-            self._call("hp_set_pool_limit", value)
-        self._pool_limit = value
+            # First, so that a block dropped from here on waits by the new limit.
+            previous, self._pool_limit = self._pool_limit, value
+            try:
+                self._return_small()
+                self._call("hp_set_pool_limit", value)
+            except BaseException:
+                self._pool_limit = previous
+                raise
 
     def pool_stats(self):
         values = [ctypes.c_int64(0) for _ in range(4)]

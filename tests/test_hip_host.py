@@ -3,6 +3,7 @@ stand-in library that hands out numbers as addresses and keeps account of them."
 
 import ctypes
 import sys
+import types
 
 import numpy as np
 import pytest
@@ -84,10 +85,10 @@ def _waiting(backend):
     return list(backend._small) + [ptr for kept in backend._kept.values() for ptr in kept]
 
 
-def _at_instruction(function, number, action):
-    """Call ``function``; before its ``number``-th instruction call ``action``.
-    False when the function has fewer instructions."""
-    code, left = function.__func__.__code__, [number]
+def _at_instruction(method, number, action, *args):
+    """Call ``method``; before its ``number``-th instruction call ``action``.
+    False when it has fewer instructions."""
+    code, left = method.__func__.__code__, [number]
 
     def trace(frame, event, arg):
         if frame.f_code is not code:
@@ -103,7 +104,7 @@ def _at_instruction(function, number, action):
 
     sys.settrace(trace)
     try:
-        function()
+        method(*args)
     finally:
         sys.settrace(None)
     return left[0] <= 0
@@ -163,3 +164,27 @@ def test_waiting_blocks_go_back_before_a_dot_fails(backend):
     backend._lib.most = 2
     with pytest.raises(RuntimeError, match="hp_dot_new"):
         backend.vector_dot(vector, vector)
+
+
+def test_no_block_waits_past_a_pool_limit(backend):
+    # A block dropped as the limit falls (by a finaliser or another thread) is
+    # judged by the new limit.
+    number, reached = 0, True
+    while reached:
+        number += 1
+        backend.pool_limit = 1 << 40
+        late = [backend.empty((100000,), np.bool_)]
+        setter = types.MethodType(type(backend).pool_limit.fset, backend)
+        reached = _at_instruction(setter, number, late.clear, 0)
+        late.clear()
+        assert backend.pool_limit == backend._lib.limit == 0
+        assert not any(backend._kept.values()), f"before instruction {number}"
+    assert number > 10
+
+
+def test_a_refused_pool_limit_changes_nothing(backend):
+    backend.pool_limit = 1 << 40
+    backend._lib.hp_set_pool_limit = lambda ctx, value: _hip_lib.HP_E_HIP
+    with pytest.raises(RuntimeError, match="hp_set_pool_limit"):
+        backend.pool_limit = 0
+    assert backend.pool_limit == 1 << 40
