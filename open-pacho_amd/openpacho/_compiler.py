@@ -560,7 +560,7 @@ class CompiledFunction:
         self._positional = _all_positional(signature)
         self.max_size = cache_size
         self._plans = OrderedDict()
-        self._quick = {}  # _quick_key of a positional call -> its key in _plans
+        self._quick = {}  # _quick_key of a positional call -> its key in _plans, for the plans there
         self._quick_names = len(self._names) if self._positional and not self.static_argnames else -1
         self._lock = RLock()
         self._hits = self._misses = 0
@@ -588,12 +588,11 @@ class CompiledFunction:
                         self._hits += 1
                         self._plans.move_to_end(key)
                         return plan, args
-        plan, bindings = self._find_plan(args, kwargs)
+        plan, bindings, key = self._find_plan(args, kwargs)
         if quick is not None:
             with self._lock:
-                if len(self._quick) >= 4 * self.max_size:
-                    self._quick.clear()
-                self._quick[quick] = self._specs(bindings)
+                if key in self._plans:  # not dropped by another thread since
+                    self._quick[quick] = key
         return plan, bindings
 
     def _find_plan(self, args, kwargs):
@@ -604,15 +603,17 @@ class CompiledFunction:
             if plan is not None:
                 self._hits += 1
                 self._plans.move_to_end(key)
-                return plan, bindings
+                return plan, bindings, key
             plan, bindings = capture_call(
                 self.python_function, args, kwargs, static_argnames=self.static_argnames, padding=self.padding
             )
             self._misses += 1
             self._plans[key] = plan
             if len(self._plans) > self.max_size:
-                self._plans.popitem(last=False)
-            return plan, bindings
+                dropped, _ = self._plans.popitem(last=False)
+                for quick in [quick for quick, of in self._quick.items() if of == dropped]:
+                    del self._quick[quick]
+            return plan, bindings, key
 
     def __call__(self, *args, **kwargs):
         # Plain NumPy inputs run the original Python function unchanged.
