@@ -348,6 +348,9 @@ def _identity(operation, dtype):
 
 def _combine(operation, dtype, left, right):
     if operation == "sum":
+        if dtype in _UNSIGNED:  # wrapping, as in hp_reduce: a signed overflow is undefined
+            u = _UNSIGNED[dtype]
+            return f"({ctype(dtype)})(({u})({left}) + ({u})({right}))"
         return f"({left}) + ({right})"
     if dtype.kind == "b":
         op = "&&" if operation == "min" else "||"

@@ -7,12 +7,14 @@ that a compiled sum rounds like the eager one and stays within the bound of
 its summation order on ordinary values.
 """
 
+import subprocess
+
 import numpy as np
 import pytest
 
 import openpacho as p
 from openpacho._hip_map_reduce import BLOCK, _column_plan, map_reduce_source
-from openpacho._hip_lowering import _Leaf
+from openpacho._hip_lowering import _Leaf, _identity
 
 # (shape, reduced axes)
 ROWS = [((5, n), (1,)) for n in (1, 3, 4, 5, 63, 64, 65, 1008, 1025, 8191, 8192, 8197)]
@@ -163,3 +165,34 @@ def test_sources_compile(shape, axes, operation, dtype):
     nodes = [(op, [0, 1, 2][: 3 if op == "where" else 2], (dtype,) * 3, dtype)]
     status, log = _compiles(map_reduce_source(shape, axes, leaves, nodes, operation, dtype)[0])
     assert status == 0, log
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.uint32, np.uint64])
+def test_integer_sums_wrap_in_constant_expressions(dtype):
+    # A constant expression may not overflow a signed type: the compiler
+    # refuses one that does.
+    from openpacho._hip_lowering import _combine, ctype
+
+    info, t = np.iinfo(dtype), ctype(dtype)
+    first, last = _identity("max", np.dtype(dtype)), _identity("min", np.dtype(dtype))
+    source = f"""
+constexpr {t} sum({t} a, {t} b) {{ return {_combine("sum", np.dtype(dtype), "a", "b")}; }}
+static_assert(sum({last}, 1) == {first} && sum({first}, {last}) == ({t})({info.min + info.max}), "");
+static_assert(sum({last}, {last}) == ({t})-2 && sum(({t})-1, 1) == 0, "");
+"""
+    done = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-x", "c++", "-"], input=source, capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("shape", [(7, 50), (3, 5000), (600, 6)])
+def test_integer_sums_wrap_in_rows_columns_and_row_programs(hip, dtype, shape):
+    host = np.random.default_rng(8).integers(np.iinfo(dtype).min, np.iinfo(dtype).max, shape, dtype=dtype, endpoint=True)
+
+    def sums(x):
+        rows = x.sum(axis=1, keepdims=True, dtype=dtype)
+        return (x + 1).sum(axis=0, dtype=dtype), (x * 3).sum(axis=1, dtype=dtype), rows, x - rows
+
+    for got, want in zip(p.compile(sums)(p.asarray(host, backend=hip)), sums(host)):
+        np.testing.assert_array_equal(p.asnumpy(got), want)
