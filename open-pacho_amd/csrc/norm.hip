@@ -144,9 +144,14 @@ __device__ __forceinline__ Pair<T> registers_to_pair(const T (&v)[N]) {
 //   kRunning a single row: every wave folds its chunks into a running pair
 //            and each workgroup writes one pair (few pairs left to merge);
 //   kWalk    rows of several chunks, enough of them to keep the chip's waves
-//            busy one row each: a wave folds its row's chunks in order and
-//            writes the norm (no pairs in memory, no merge launch; 16384 rows
-//            of 8190 float32: 146 -> 84 us).
+//            busy one row each: a wave walks its row and writes the norm (no
+//            pairs in memory, no merge launch; 16384 rows of 8190 float32:
+//            146 -> 84 us). Lane i keeps the pair of chunk i; 64 of them meet
+//            in a butterfly, and the butterflies' results in order: the order
+//            of norm_merge_kernel, bit for bit, for rows of at most kWalkChunks
+//            chunks (one pair per thread there), so the error of a norm does
+//            not depend on the number of rows. Added one after the other, 128
+//            chunks had three times that error.
 // kVector: nearly every chunk is whole and 16-byte aligned (65536 rows of 4096
 // float32: 154 us; the guarded loads of the other form 168 us). Otherwise a
 // wave reads groups of 16 bytes at element alignment, all of a chunk's before
@@ -156,6 +161,7 @@ __device__ __forceinline__ Pair<T> registers_to_pair(const T (&v)[N]) {
 constexpr int kFinal = 0, kPairs = 1, kRunning = 2, kWalk = 3;
 // Rows at which kWalk gives every compute unit 16 waves.
 constexpr int64_t kWalkRows = 4096;
+constexpr int64_t kWalkChunks = kBlock;
 // Longest row of norm_short_kernel: 16 elements a lane of one wave.
 constexpr int64_t kShort = 1024;
 
@@ -235,7 +241,8 @@ __global__ __launch_bounds__(kBlock) void norm_rows_kernel(const T* __restrict__
   const int64_t units = MODE == kWalk ? outer : outer * chunks;
   const int64_t stride = int64_t(gridDim.x) * (kBlock / 64);
   Pair<T> running = {T(-INFINITY), T(0)};
-  int64_t walked = 0;  // chunks of the current row already in `running` (kWalk)
+  Pair<T> mine = running;  // kWalk: the pair of chunk `walked` - 64 k = lane
+  int64_t walked = 0;      // kWalk: chunks of the current row already read
   for (int64_t g = int64_t(blockIdx.x) * (kBlock / 64) + wave; g < units;) {
     const int64_t o = MODE == kWalk ? g : g / chunks, ch = MODE == kWalk ? walked : g - o * chunks;
     const int64_t begin = ch * kLen;
@@ -262,10 +269,13 @@ __global__ __launch_bounds__(kBlock) void norm_rows_kernel(const T* __restrict__
     }
     const Pair<T> p = registers_to_pair<T, N>(v);
     if (MODE == kWalk) {
-      running = merge(running, p);
-      if (++walked < chunks) continue;
+      if (lane == int(walked % 64)) mine = p;
+      if (++walked % 64 != 0 && walked < chunks) continue;
+      running = merge(running, wave_merge(mine));
+      mine = {T(-INFINITY), T(0)};
+      if (walked < chunks) continue;
       if (lane == 0) out[o] = finish(running);
-      running = {T(-INFINITY), T(0)};
+      running = mine;
       walked = 0;
     } else if (MODE == kRunning) {
       running = merge(running, p);
@@ -451,7 +461,8 @@ RowPlan plan_rows(hp_ctx* ctx, const T* x, int64_t outer, int64_t reduced) {
   }
   plan.vector = reinterpret_cast<uintptr_t>(x) % 16 == 0 && (reduced * int64_t(sizeof(T))) % 16 == 0 &&
                 (reduced % chunk_len<T>() == 0 || plan.chunks > 8);
-  plan.mode = plan.chunks == 1 ? kFinal : (outer == 1 ? kRunning : (outer >= kWalkRows ? kWalk : kPairs));
+  const bool walk = outer >= kWalkRows && plan.chunks <= kWalkChunks;
+  plan.mode = plan.chunks == 1 ? kFinal : (outer == 1 ? kRunning : (walk ? kWalk : kPairs));
   const int64_t units = plan.mode == kWalk ? outer : outer * plan.chunks;
   // Enough resident waves to keep HBM busy; the grid loops over the rest.
   const int64_t resident = int64_t(ctx->compute_units) * kResidentGroupsPerCU;

@@ -40,3 +40,25 @@ def test_row_norms(hip, rows, length, dtype):
     np.testing.assert_allclose(got[finite], want[finite].astype(np.float64), rtol=bound * np.finfo(dtype).eps / 2)
     assert got[3] == np.inf and np.isnan(got[4]) and np.isnan(got[5])
     assert got[2] == 0 and not np.signbit(got[2])
+
+
+# Several chunks of a wave (4096 float32 or 2048 float64), around one, two and four
+# butterflies of 64 of them.
+LONG = [(np.float32, n) for n in (8190, 4096 * 63 + 5, 4096 * 64, 4096 * 65, 4096 * 127 + 4)]
+LONG += [(np.float64, n) for n in (2 * 2048 + 2, 64 * 2048, 129 * 2048 + 1, 255 * 2048 + 8)]
+
+
+@pytest.mark.parametrize("dtype,length", LONG)
+def test_a_norm_does_not_depend_on_the_number_of_rows(hip, dtype, length):
+    # 4096 rows are walked by a wave each; fewer leave pairs to a merge kernel.
+    rows = 4096
+    x = p.random.default_rng(length, backend=hip).normal(0.0, 1.0, (rows, length), dtype=np.dtype(dtype).name)
+    walked = p.asnumpy(p.linalg.norm(x, axis=1))
+    few = x[: rows - 1000]
+    del x
+    np.testing.assert_array_equal(p.asnumpy(p.linalg.norm(few, axis=1)), walked[: rows - 1000])
+    exact = np.linalg.norm(p.asnumpy(few[:20]).astype(np.longdouble), axis=1)
+    # A lane's chain of at most 65 fused squares, the wave's 6 steps, the 6 of
+    # the butterfly over chunks and the merges of 4; the root halves the error.
+    bound = (65 + 6 + 6 + 4) / 2 + 1
+    np.testing.assert_allclose(walked[:20], exact.astype(np.float64), rtol=bound * np.finfo(dtype).eps / 2)
