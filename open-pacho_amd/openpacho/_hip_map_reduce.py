@@ -269,13 +269,45 @@ def _folded_rows(m, width):
     return 1, False
 
 
+# Batches of a float sum that may join one accumulator one after the other.
+LONGEST_CHAIN = 4
+
+
+def _cascade(m, width, levels):
+    """Sources that declare, add to and close `levels` partial sums of `carry`s:
+    level l holds the sum of 2^l of them and is full where bit l of their count
+    is set, so that every sum is of two of the same size. A chain of them adds
+    an error of its length's root: 4095 rows of 524288 float32 columns, 512
+    batches in one chain, had 7 times the error of lanes that meet in a tree
+    (squares of normal values, rms), and with levels 0.93 times (300 to 262144
+    rows: 0.91 to 1.10, which the sample does not tell apart). The count is the
+    same for all threads of a wave that still add, so the branches cost a
+    scalar test each: 4095 x 262144 float32 took 672 us in one chain and 648
+    with levels, 100003 x 1025 68.4 and 68.1, 65536 x 4096 167 and 165."""
+    if not levels:
+        return [], [], []
+    each = f"_Pragma(\"unroll\") for (int v = 0; v < {width}; ++v)"
+    declare = [f"{m.acc} carry[{width}], level[{levels}][{width}];", "unsigned count = 0;"]
+    join, close = [], ["}" * (levels - 1)]
+    for l in range(levels):
+        keep = f"{each} level[{l}][v] = carry[v];"
+        if l == levels - 1:
+            join.append(keep)
+        else:
+            add = f"{each} carry[v] = {m.combine(f'level[{l}][v]', 'carry[v]')};"
+            join += [f"if (!(count & {1 << l}U)) {{ {keep} }} else {{", f"  {add}"]
+    join += [*close, "++count;"]
+    close = [f"if (count & {1 << l}U) {{ {each} acc[v] = {m.combine('acc[v]', f'level[{l}][v]')}; }}" for l in range(levels)]
+    return declare, join, close
+
+
 def _columns(m):
     """A workgroup owns a block of columns and a chunk of rows; a thread reads
     `width` adjacent columns of every step-th row, eight rows (16 of one
-    column) in flight. Each batch folds on its own, in pairs, before it joins
-    the accumulator, so the chain of a sum is rows / 8 long; the rows of a step
-    meet in LDS in a fixed tree. Leaves that vary along inner only are read
-    once. Bound by HBM: where rows are whole vectors a thread takes 16 bytes
+    column) in flight. Each batch folds on its own, in pairs; the batches of a
+    float sum then meet in pairs too (_cascade), those of other reductions in
+    one accumulator; the rows of a step meet in LDS in a fixed tree. Leaves
+    that vary along inner only are read once. Bound by HBM: where rows are whole vectors a thread takes 16 bytes
     with the nontemporal hint (100003 x 1024 float32: 67 us, 6.1 TB/s, against
     78 us without the hint). Other rows are folded (_folded_rows): 32 rows of
     1025 float32 are one row of 32800 columns that starts on a line, whose
@@ -314,7 +346,10 @@ def _columns(m):
         arguments = "".join(", " + names.get(m.access[k], "s%d") % k for k in given)
         return f"mapped(first + r * {inner}LL + {j * step * inner + v}LL{arguments})"
 
-    def fold(count):
+    most = -(-rows // (batch * step))  # batches of a thread
+    levels = most.bit_length() if m.operation == "sum" and m.acc_dtype.kind == "f" and most > LONGEST_CHAIN else 0
+
+    def fold(count, into="acc"):
         lines = []
         for v in range(width):
             lines += ["{", *(f"  {m.acc} some{j} = {value(j, v)};" for j in range(count))]
@@ -323,9 +358,11 @@ def _columns(m):
                 for j in range(0, count - apart, 2 * apart):
                     lines.append(f"  some{j} = {m.combine(f'some{j}', f'some{j + apart}')};")
                 apart *= 2
-            lines += [f"  acc[{v}] = {m.combine(f'acc[{v}]', 'some0')};", "}"]
+            joined = m.combine(f"acc[{v}]", "some0") if into == "acc" else "some0"
+            lines += [f"  {into}[{v}] = {joined};", "}"]
         return lines
 
+    declare, join, close = _cascade(m, width, levels)
     tree = f"""
   for (int n = {step}; n > 1;) {{
     const int half = (n + 1) / 2;
@@ -359,12 +396,12 @@ def _columns(m):
 #pragma unroll
   for (int v = 0; v < {width}; ++v) acc[v] = {m.identity};
   if (active) {{
-    {_lines(constants, 4)}
+    {_lines(constants + declare, 4)}
     long long r = begin + row;
     for (; r + {(batch - 1) * step} < whole; r += {batch * step}) {{
       {_lines([line for j in range(batch) for line in loads(j)], 6)}
       {FENCE}
-      {_lines(fold(batch), 6)}
+      {_lines(fold(batch, "carry") + join if levels else fold(batch), 6)}
     }}
     for (; r < whole; r += {step}) {{
       {_lines(loads(0), 6)}
@@ -378,6 +415,7 @@ def _columns(m):
         }}
       }}
     }}
+    {_lines(close, 4)}
   }}{tree}
   if (active && row == 0) {{
     for (int v = 0; v < {width}; ++v) out[(o * {chunks}LL + chunk) * {inner}LL + col + v] = acc[v];

@@ -196,3 +196,26 @@ def test_integer_sums_wrap_in_rows_columns_and_row_programs(hip, dtype, shape):
 
     for got, want in zip(p.compile(sums)(p.asarray(host, backend=hip)), sums(host)):
         np.testing.assert_array_equal(p.asnumpy(got), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", [(4095, 262144), (8191, 65537), (100003, 36), (70001, 1025), (300, 4096), (41, 9)])
+def test_column_sums_keep_what_a_long_chain_would_lose(hip, dtype, shape):
+    # After a first row of half the type's digits beyond one, each 1 is less
+    # than half a unit in the last place: an accumulator that took the rows, or
+    # pairs and fours of them, one after the other would drop them all. Sums of
+    # two equal parts drop what comes before the parts reach that unit.
+    digits = np.finfo(dtype).nmant
+    first = 2.0 ** (digits + 5)  # a unit in the last place is 32
+    weights = np.ones((shape[0], 1), dtype)
+    weights[0] = first
+    compiled = p.compile(lambda x, w: (x * w).sum(axis=0))
+    got = p.asnumpy(compiled(p.ones(shape, dtype=dtype, backend=hip), p.asarray(weights, backend=hip)))
+    exact = first + (shape[0] - 1)
+    # On the way of the first row: 8 rows of a batch, the levels of at most
+    # rows / 8 batches, up to 7 single rows, the tree of a step's rows and the
+    # merge of the partials (their own chain of at most 16 and a tree): half a
+    # unit for each sum.
+    bound = (3 + np.log2(max(shape[0], 8)) + 7 + 8 + 16 + 8) * 16
+    assert np.all(np.abs(got.astype(np.longdouble) - exact) <= bound), (got[0] - exact, bound)
