@@ -62,3 +62,17 @@ def test_a_norm_does_not_depend_on_the_number_of_rows(hip, dtype, length):
     # the butterfly over chunks and the merges of 4; the root halves the error.
     bound = (65 + 6 + 6 + 4) / 2 + 1
     np.testing.assert_allclose(walked[:20], exact.astype(np.float64), rtol=bound * np.finfo(dtype).eps / 2)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("length", [17, 49, 64, 65, 257, 1024])
+def test_short_rows_keep_squares_below_half_a_unit(hip, length, dtype):
+    # After a leading 1 each square is just under half a unit in the last place:
+    # one chain of a lane's 16 elements drops 15 of them (7.5 units of u for the
+    # root). Of four chains the one with the 1 drops at most 4; sums of parts
+    # that grew apart from it are off by half a unit each, 2 + 6 of them, and so is the root.
+    host = np.full((70, length), 0.99 * np.sqrt(np.finfo(dtype).eps / 2), dtype)
+    host[:, 0] = 1
+    got = p.asnumpy(p.linalg.norm(p.asarray(host, backend=hip), axis=1))
+    exact = np.linalg.norm(host.astype(np.longdouble), axis=1)
+    np.testing.assert_allclose(got, exact.astype(np.float64), rtol=(4 + 2 + 6 + 1) / 4 * np.finfo(dtype).eps)
