@@ -28,7 +28,7 @@ import numpy as np
 
 from . import _hip_lowering as source_
 from ._compiler import ELEMENTWISE, Step
-from ._hip_map_reduce import WAVES, row_lanes
+from ._hip_map_reduce import CHUNK, COMPUTE_UNITS, WAVES, row_lanes
 
 # Operations cheap enough to repeat in every reader of a value.
 CHEAP = frozenset(
@@ -40,6 +40,21 @@ MOST_MERGED = 8  # outputs of a merged launch
 MOST_ARGUMENTS = 256  # operands of its members together: far below what a packed launch takes
 SMALL = 1 << 16  # elements up to which a step may run later than the plan has it
 MOST_REGISTERS = 160  # 32-bit registers of row values per lane
+# By operation and whether it is in float32 or wider. What one element adds to
+# the time of a lane that has its SIMD to itself, in us (the rest: next to
+# nothing), fitted to rows of 4000 to 16384 elements.
+LANE_TIME = {
+    ("power", 4): 0.55, ("sin", 4): 0.1, ("cos", 4): 0.1, ("tanh", 4): 0.1,
+    ("power", 8): 0.55, ("tanh", 8): 0.33, ("sin", 8): 0.2, ("cos", 8): 0.2, ("log", 8): 0.2, ("exp", 8): 0.05,
+}
+LAUNCH_TIME = 4.0  # us that a launch less saves a call
+# Elements that fit the compiler's limit on a lane's unrolled code; past it the
+# row goes to scratch memory (sin over 16384 x 16384 float32: 531 us in steps,
+# 1183 in a program of 64 elements a lane; 56 still fit).
+MOST_UNROLLED = {
+    ("sin", 4): 56, ("cos", 4): 56, ("tanh", 4): 192,
+    ("sin", 8): 64, ("cos", 8): 64, ("power", 8): 64, ("tanh", 8): 96, ("log", 8): 192,
+}
 
 
 class Launch(NamedTuple):
@@ -214,9 +229,37 @@ def _row_program(steps, begin, end, space, kept):
         return None
     if sum(a == "full" for a in access) > 4:
         return None
-    source = _row_source(run, inside, outputs, args, leaves, access, space, lanes, groups)
     grid = -(-space.outer // (source_.BLOCK // lanes))
+    if not _serves(run, {id(a) for a in args} | set(inside), space, groups * source_.VECTOR, grid):
+        return None
+    source = _row_source(run, inside, outputs, args, leaves, access, space, lanes, groups)
     return Launch(tuple(outputs), tuple(args), _Kernel(source, "pacho_rows", grid))
+
+
+def _serves(run, stored, space, elements, grid):
+    """Whether a program of `elements` a lane and `grid` workgroups is as fast
+    as its steps. Few long rows leave most of the chip to the steps alone, whose
+    lanes take 16 elements each: with operations that keep a lane busy that is
+    worth more than the launches (x ** 1.7 and its maximum over 4 x 8192
+    float32, alone: 31.4 us against 27.4; tanh over 4 x 8192 float64 27.3
+    against 24.6, over 4 x 4000 22.5 against 23.4). The gap closes as workgroups
+    share compute units, at four of them altogether (1024 x 8192 float64, power:
+    59.7 against 64.1)."""
+    time = 0.0
+    for step in run:
+        fused = step.kind == "fused"
+        root = step.node if fused else step.node.inputs[0]
+        if (fused and space.access(root.shape) != "full") or (not fused and id(root) in stored):
+            continue
+        group, _ = _collect(root, stored - {id(root)})
+        kinds = [(node.op, 4 if node.dtype == np.float32 else 8) for node in group]
+        if sum(elements / MOST_UNROLLED[kind] for kind in kinds if kind in MOST_UNROLLED) > 1:
+            return False
+        time += sum(LANE_TIME.get(kind, 0.0) for kind in kinds)
+    launches = len(run) - 1 + sum(step.kind != "fused" and space.reduced > CHUNK for step in run)
+    idle = max(0.0, 1 - grid / (4 * COMPUTE_UNITS))
+    more = elements - source_.ELEMENTS_PER_THREAD * source_.VECTOR
+    return time * more * idle <= LAUNCH_TIME * launches
 
 
 def _row_source(run, inside, outputs, args, leaves, access, space, lanes, groups):

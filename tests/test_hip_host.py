@@ -1,13 +1,19 @@
 """Host side of HIPBackend without a device: its blocks and their lifetime on a
-stand-in library that hands out numbers as addresses and keeps account of them."""
+stand-in library that hands out numbers as addresses and keeps account of them,
+and the launches that it arranges a plan into."""
 
 import ctypes
+import re
+import shutil
+import subprocess
 import sys
 import types
+from pathlib import Path
 
 import numpy as np
 import pytest
 
+import openpacho as p
 from openpacho import _hip, _hip_lib
 from openpacho._array import ndarray
 from openpacho.backends import DeviceInfo
@@ -188,3 +194,63 @@ def test_a_refused_pool_limit_changes_nothing(backend):
     with pytest.raises(RuntimeError, match="hp_set_pool_limit"):
         backend.pool_limit = 0
     assert backend.pool_limit == 1 << 40
+
+
+# ---- plans -------------------------------------------------------------------------
+
+
+def _launches(backend, function, shape, dtype):
+    """The launches of a compiled function of one array."""
+    plan, _ = p.compile(function)._plan((p.empty(shape, dtype=dtype, backend=backend),), {})
+    return plan._launches
+
+
+def _and_squares(function):
+    def result(x):
+        y = function(x)
+        return y, (y * y).sum(axis=-1)
+
+    return result
+
+
+def _softmax(x):
+    e = np.exp(x - x.max(axis=-1, keepdims=True))
+    return e / e.sum(axis=-1, keepdims=True)
+
+
+POWER, TANH, SIN = (_and_squares(f) for f in (lambda x: x**1.7, np.tanh, np.sin))
+# Rows that one launch serves, and rows that stay steps: few long ones of
+# operations that keep a lane busy, at 16, 32 and 64 elements a lane and around
+# the workgroups that fill the chip; and any whose unrolled code is too long.
+ONE = [(POWER, (4, 4096), "f4"), (POWER, (4, 4096), "f8"), (POWER, (1024, 8192), "f4"), (POWER, (1024, 8192), "f8")]
+ONE += [(TANH, (4, 4096), "f8"), (TANH, (256, 8192), "f8"), (TANH, (4, 16384), "f4"), (SIN, (4, 8192), "f8")]
+ONE += [(SIN, (4, 8192), "f4"), (SIN, (4096, 14336), "f4"), (_softmax, (4, 16384), "f4"), (_softmax, (4, 8192), "f8")]
+STEPS = [(POWER, (4, 8192), "f4"), (POWER, (512, 8192), "f4"), (POWER, (64, 8192), "f8"), (POWER, (256, 16384), "f4"), (TANH, (64, 8192), "f8")]
+STEPS += [(SIN, (4, 16384), "f4"), (SIN, (16384, 16384), "f4"), (_and_squares(lambda x: np.sin(x) + np.cos(x)), (4096, 10240), "f8")]
+
+
+@pytest.mark.parametrize("function,shape,dtype", ONE)
+def test_rows_that_one_launch_serves(backend, function, shape, dtype):
+    assert len(_launches(backend, function, shape, dtype)) == 1
+
+
+@pytest.mark.parametrize("function,shape,dtype", STEPS)
+def test_rows_that_stay_steps(backend, function, shape, dtype):
+    assert len(_launches(backend, function, shape, dtype)) == 2
+
+
+def test_long_rows_stay_in_registers(tmp_path, backend):
+    if not (shutil.which("hipcc") or Path("/opt/rocm/bin/hipcc").exists()):
+        pytest.skip("hipcc not available")
+    import build
+
+    both = _and_squares(lambda x: np.sin(x) + np.cos(x))
+    for function, shape, dtype in [(SIN, (4096, 14336), "f4"), (both, (4096, 8192), "f8"), (TANH, (4096, 10240), "f8")]:
+        (launch,) = _launches(backend, function, shape, dtype)
+        source = tmp_path / "rows.hip"
+        source.write_text("#include <hip/hip_runtime.h>\n" + launch.payload.source)
+        command = [build.hipcc(), "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt"]
+        command += ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "--cuda-device-only", "-c"]
+        command += ["-Rpass-analysis=kernel-resource-usage", str(source), "-o", str(tmp_path / "rows.o")]
+        remarks = subprocess.run(command, capture_output=True, text=True, check=True).stderr
+        assert re.search(r"ScratchSize \[bytes/lane\]: 0\b", remarks), (shape, dtype)
