@@ -285,6 +285,17 @@ int hp_event_destroy(hp_event* event);
  * Replaces: the fake driver failures of tests/test_cuda_arguments.py:123-183. */
 int hp_debug_fail_next(hp_ctx* ctx, int count);
 
+/* Have every float product of this context take the LDS-staged kernels
+ * (on != 0), also those that the direct kernels would serve, so that tests
+ * reach all of the staged ones. */
+int hp_debug_staged_products(hp_ctx* ctx, int on);
+
+/* The direct kernels' plan of a product (every extent > 0) on a GPU of
+ * `compute_units`, without a device: plan[0] x plan[1] outputs per tile and
+ * plan[2] splits of K; plan[0] == 0: the staged kernels take it. */
+int hp_debug_direct_plan(int compute_units, int dtype, int64_t m, int64_t n, int64_t k, int64_t batch,
+                         int64_t* plan);
+
 #ifdef __cplusplus
 }
 #endif

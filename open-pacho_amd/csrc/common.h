@@ -87,6 +87,7 @@ struct hp_ctx {
   size_t live_bytes = 0;
   size_t pool_limit = 0;
   int fail_next = 0;
+  bool staged_products = false;  // hp_debug_staged_products
 };
 
 namespace hp {

@@ -19,7 +19,7 @@ __global__ __launch_bounds__(256) void zero_kernel(T* __restrict__ out, int64_t 
 void run(hp_ctx* ctx, int dtype, bool ta, bool tb, const void* a, const void* b, void* c, int64_t m, int64_t n,
          int64_t k, const hpgemm::BatchDesc& bd, int64_t batch) {
   const hpgemm::DirectPlan direct = hpgemm::direct_plan(ctx->compute_units, dtype, m, n, k, batch);
-  if (direct.fi > 0) {
+  if (direct.fi > 0 && !ctx->staged_products) {
     (dtype == HP_F32 ? hpgemm::direct_f32 : hpgemm::direct_f64)(ctx, direct, ta, tb, a, b, c, m, n, k, bd, batch);
     return;
   }
@@ -254,6 +254,25 @@ int hp_gemm_layout(hp_ctx* ctx, int dtype, const void* a, const void* b, void* c
     require(a != nullptr && b != nullptr, "null input");
     hpgemm::BatchDesc bd{};
     run(ctx, dtype, transpose_a != 0, transpose_b != 0, a, b, c, m, n, k, bd, 1);
+  });
+}
+
+int hp_debug_staged_products(hp_ctx* ctx, int on) {
+  return guarded([&] {
+    hp::enter(ctx);
+    ctx->staged_products = on != 0;
+  });
+}
+
+int hp_debug_direct_plan(int compute_units, int dtype, int64_t m, int64_t n, int64_t k, int64_t batch,
+                         int64_t* plan) {
+  return guarded([&] {
+    require(dtype == HP_F32 || dtype == HP_F64, "gemm supports float32 and float64");
+    require(compute_units > 0 && m > 0 && n > 0 && k > 0 && batch > 0 && plan != nullptr, "not a product");
+    const hpgemm::DirectPlan p = hpgemm::direct_plan(compute_units, dtype, m, n, k, batch);
+    plan[0] = 16 * p.fi;
+    plan[1] = 16 * p.fj;
+    plan[2] = p.splits;
   });
 }
 

@@ -73,6 +73,8 @@ PROTOTYPES = {
     "hp_event_elapsed_ms": [_ptr, _ptr, ctypes.POINTER(ctypes.c_float)],
     "hp_event_destroy": [_ptr],
     "hp_debug_fail_next": [_ptr, _i32],
+    "hp_debug_staged_products": [_ptr, _i32],
+    "hp_debug_direct_plan": [_i32, _i32, _i64, _i64, _i64, _i64, _ptr],
 }
 _RESTYPES = {"hp_last_error": ctypes.c_char_p, "hp_version": ctypes.c_char_p}
 

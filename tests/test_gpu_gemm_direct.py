@@ -65,3 +65,17 @@ def test_direct_batches_broadcast(hip, dtype, left, right):
     k = left[-1]
     bound = (k + 1) * np.finfo(dtype).eps / 2 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
     assert np.all(np.abs(got - a.astype(np.longdouble) @ b.astype(np.longdouble)) <= bound)
+
+
+# Shapes for every tile, with and without a K split (test_gemm_plans.py checks that
+# the set is complete): narrow extents below, at and above one block of 16.
+TILE_SHAPES = [(9, 8200, 300), (16, 4100, 300), (17, 4100, 65), (5, 700, 4099), (16, 700, 4099), (31, 700, 4099)]
+TILE_SHAPES += [(n, m, k) for m, n, k in TILE_SHAPES]
+TILE_SHAPES += [(5, 9, 4099), (33, 2050, 17), (64, 129, 4099), (64, 4100, 17), (64, 129, 8192), (129, 64, 8192)]
+TILE_SHAPES += [(8192, 33, 17), (4100, 70, 64), (300, 70, 8192), (64, 8200, 17), (8200, 64, 17), (64, 300, 8192)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n,k", TILE_SHAPES)
+def test_every_direct_tile_in_every_layout(hip, dtype, m, n, k):
+    test_direct_products_in_every_layout(hip, dtype, m, n, k)
