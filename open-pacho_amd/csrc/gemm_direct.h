@@ -21,7 +21,7 @@
 // Rows past the end read clamped addresses and feed outputs that are not
 // stored; k past the end reads as +0 for both operands (one guarded slice).
 //
-// Bound by: MFMA issue in the 64 x 64 tile (64 MFMAs per 8 or 16 KB of loads;
+// Bound by: MFMA issue in the 64 x 64 tile (fp32; 64 MFMAs per 8 KB of loads;
 // DEPTH slices of registers keep the next loads in flight behind them), by the
 // reads of the wide operand in the 16- and 32-row tiles.
 #pragma once

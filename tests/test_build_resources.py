@@ -7,7 +7,7 @@ than any test of results shows (a spilling fp64 GEMM loader once cost
 4096^2 x 4095 fp64 12 points of peak with every test green), so the budgets
 are checked here: no fp32 GEMM, GEMV, norm, reduction or RNG kernel spills,
 fp64 GEMM kernels stay within their known spills, and the GEMMs keep two
-waves per SIMD. Skipped when the library has not been built in this tree.
+waves per SIMD (one, without a spill, in the fp64 direct products). Skipped when the library has not been built in this tree.
 The GEMM units are also compiled to assembly here, to check the order of
 their LDS reads, barriers and waits.
 """
@@ -63,6 +63,16 @@ def test_fp64_gemm_spills_stay_within_known_limits(resources):
             assert r.get("VGPRs Spill", 0) <= limit, (unit, name, r)
             if "f646kernel" in name:
                 assert r["Occupancy [waves/SIMD]"] >= 2, (unit, name, r)
+
+
+@pytest.mark.parametrize("unit,waves", [("gemm_direct_f32", 2), ("gemm_direct_f64", 1)])
+def test_direct_gemm_kernels_do_not_spill_and_keep_their_waves(resources, unit, waves):
+    kernels = _kernels(resources, unit)
+    assert len(kernels) > 20, unit
+    for name, r in kernels.items():
+        assert r.get("VGPRs Spill", 0) == 0 and r.get("SGPRs Spill", 0) == 0, (unit, name, r)
+        assert r.get("ScratchSize [bytes/lane]", 0) == 0, (unit, name, r)
+        assert r["Occupancy [waves/SIMD]"] >= waves, (unit, name, r)
 
 
 @pytest.mark.parametrize("unit", ["gemv", "norm", "reduce", "philox", "copy", "gemm"])
