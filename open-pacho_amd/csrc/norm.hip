@@ -156,14 +156,17 @@ __device__ __forceinline__ Pair<T> registers_to_pair(const T (&v)[N]) {
 // float32: 154 us; the guarded loads of the other form 168 us). Otherwise a
 // wave reads groups of 16 bytes at element alignment, all of a chunk's before
 // the first is used (22544 rows of 3547: 61 us element by element, 48 us like
-// this); rows of up to half a chunk take half the loads
-// (LOADS = kLoads / 2), so that short rows do not pay for empty registers.
+// this); fp32 rows of up to half a chunk (kHalf) take half the loads
+// (LOADS = kLoads / 2), so that they do not pay for empty registers. In fp64
+// half a chunk is no longer than kShort, whose rows have their own kernel.
 constexpr int kFinal = 0, kPairs = 1, kRunning = 2, kWalk = 3;
 // Rows at which kWalk gives every compute unit 16 waves.
 constexpr int64_t kWalkRows = 4096;
 constexpr int64_t kWalkChunks = kBlock;
 // Longest row of norm_short_kernel: 16 elements a lane of one wave.
 constexpr int64_t kShort = 1024;
+template <typename T>
+constexpr bool kHalf = chunk_len<T>() / 2 > kShort;
 
 // The `len` elements at `base`, `lanes` lanes taking a group of 16 bytes each
 // in turn; the last len % width elements, one a lane, come in v's last entry.
@@ -495,9 +498,14 @@ void run_rows(hp_ctx* ctx, const RowPlan& plan, const T* x, T* out, int64_t oute
     if (plan.vector) norm_rows_kernel<T, kLoads, true, MODE_><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks); \
     else norm_rows_kernel<T, kLoads, false, MODE_><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks);            \
   } while (0)
-  if (plan.mode == kFinal && reduced <= chunk_len<T>() / 2)
-    norm_rows_kernel<T, kLoads / 2, false, kFinal><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks);
-  else if (plan.mode == kFinal) PACHO_NORM_LAUNCH(kFinal);
+  if constexpr (kHalf<T>) {
+    if (plan.mode == kFinal && reduced <= chunk_len<T>() / 2) {
+      norm_rows_kernel<T, kLoads / 2, false, kFinal><<<grid, kBlock, 0, ctx->stream>>>(x, target, outer, reduced, chunks);
+      hp::check_launch("norm_rows");
+      return;
+    }
+  }
+  if (plan.mode == kFinal) PACHO_NORM_LAUNCH(kFinal);
   else if (plan.mode == kRunning) PACHO_NORM_LAUNCH(kRunning);
   else if (plan.mode == kWalk) PACHO_NORM_LAUNCH(kWalk);
   else PACHO_NORM_LAUNCH(kPairs);
