@@ -75,38 +75,33 @@ def test_folded_rows_are_exact_on_small_integers(hip, shape, axes, dtype):
         np.testing.assert_array_equal(p.asnumpy(most), np.max(host - other, axis=axes))
 
 
-def _touched(shape, axes, leaf, dtype):
-    """How often the column kernel's index arithmetic reads each element, and the partials it leaves."""
-    from openpacho._hip_map_reduce import _Mapped, _folded_rows
+# Rows of each shape that become one, by the rule: as many as start on a line
+# where 64 long rows are left, on a vector where 16 are; one where single columns
+# need no partials, and where rows are whole vectors. (4- and 8-byte elements)
+FOLDS = [(1, 1), (1, 1), (4, 2), (4, 16), (4, 16), (4, 16), (32, 16), (32, 16), (32, 16), (32, 16)]
+FOLDS += [(32, 16), (16, 1), (16, 1), (32, 16), (32, 16)]
 
-    m = _Mapped(shape, axes, [_Leaf(False, dtype, shape), _Leaf(False, dtype, leaf)], [("add", [0, 1], (dtype,) * 2, dtype)], "sum", dtype)
+
+@pytest.mark.parametrize("case,folds", list(zip(FOLDED, FOLDS, strict=True)))
+@pytest.mark.parametrize("dtype", ["f4", "f8"])
+def test_folded_rows_start_on_lines_or_vectors_and_their_plans_cover_them(case, folds, dtype):
+    # What the kernel then reads is compared on the device (the exact sums above).
+    from openpacho._hip_map_reduce import MOST_PARTIAL_BYTES, _folded_rows, _Mapped
+
+    (shape, axes), dtype = case, np.dtype(dtype)
+    leaves = [_Leaf(False, dtype, shape), _Leaf(False, dtype, shape[-1:])]
+    m = _Mapped(shape, axes, leaves, [("add", [0, 1], (dtype,) * 2, dtype)], "sum", dtype)
     width = 16 // dtype.itemsize
     folded, lines = _folded_rows(m, width)
+    assert folded == folds[dtype.itemsize // 8]
     if folded == 1:
-        return folded, None
-    inner, total, reduced = folded * m.inner, m.reduced * m.inner, -(-m.reduced // folded)
+        return
+    inner, reduced = folded * m.inner, -(-m.reduced // folded)
+    assert inner * dtype.itemsize % (128 if lines else 16) == 0 and reduced >= (64 if lines else 16)
+    assert m.outer * inner * dtype.itemsize <= MOST_PARTIAL_BYTES
     across, blocks, step, rows, chunks = _column_plan(m.outer, reduced, inner, width, dtype.itemsize, 8 if lines else 1)
-    touched = np.zeros(total, int)
-    for col in range(0, inner, width):
-        for chunk in range(chunks):
-            end = min((chunk + 1) * rows, reduced)
-            whole = min((total - col - width + inner) // inner, end)
-            r = np.arange(chunk * rows, end)
-            for v in range(width):
-                at = r * inner + col + v
-                assert np.all(at[r < whole] < total) and np.sum(r >= whole) <= 1
-                touched[at[at < total]] += 1
     assert across * step <= BLOCK and (blocks - 1) * across * width < inner <= blocks * across * width
-    return folded, touched
-
-
-@pytest.mark.parametrize("shape,axes", FOLDED)
-@pytest.mark.parametrize("dtype", ["f4", "f8"])
-def test_folded_rows_read_every_element_once(shape, axes, dtype):
-    folded, touched = _touched(shape, axes, shape[-1:], np.dtype(dtype))
-    if shape[0] >= 2048 and shape[-1] % 2:
-        assert folded > 1
-    assert touched is None or np.all(touched == 1)
+    assert rows % step == 0 and (chunks - 1) * rows < reduced <= chunks * rows
 
 
 @pytest.mark.gpu
