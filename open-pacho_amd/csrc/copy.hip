@@ -78,33 +78,37 @@ struct Packed {
   typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
 };
 
-// Elements in order of dst: a thread moves kGroups runs of V consecutive dst
-// elements (16 bytes for 4- and 8-byte words). A run inside one innermost row
-// takes one index computation, one vector load when the row is contiguous in
-// src (UNIT) and one vector store; a run that crosses a row end or the end of
-// dst goes element by element. Strided rows (UNIT = 0) load V words and rely
-// on the caches for the parts of lines that neighbours use.
-constexpr int kGroups = 4;
-
-template <typename T, int V, bool UNIT, typename I>
+// Elements in order of dst: a thread moves G runs of V consecutive dst elements
+// (16 bytes for 4- and 8-byte words), all loads before the first store. A run
+// inside one innermost row takes one index computation, and one vector load
+// when the row is contiguous in src (UNIT); a run that crosses a row end takes
+// an index computation per element. Either way it is one vector store: runs
+// are contiguous in dst. Strided rows (UNIT = 0) load V words and rely on the
+// caches for the parts of lines that neighbours use. (Runs that crossed went
+// element by element, each load behind the store before it, and every wave of
+// an odd row length has such runs: columns 1 to 9 of 3000000 x 11 float32
+// 68.6 us, every seventh column 55.5, a 3 x 1080 x 1920 image to channels last
+// in float64 22.5; now 37.7, 25.9 and 17.)
+template <typename T, int V, bool UNIT, typename I, int G>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ src, T* __restrict__ dst, I count,
                                                           int rank, Strided layout) {
   using Vec = typename Packed<T, V>::type;
   const I length = I(layout.shape[rank - 1]);
   const int64_t step = UNIT ? 1 : layout.strides[rank - 1];
-  Vec v[kGroups];
-  I at[kGroups];
-  bool whole[kGroups];
+  Vec v[G];
+  I at[G];
 #pragma unroll
-  for (int g = 0; g < kGroups; ++g) {
-    const I i = ((I(blockIdx.x) * kGroups + g) * 256 + threadIdx.x) * V;
+  for (int g = 0; g < G; ++g) {
+    const I i = ((I(blockIdx.x) * G + g) * 256 + threadIdx.x) * V;
     at[g] = i;
-    whole[g] = false;
     if (i >= count) continue;
     I col;
     const I row = split<I>(i, layout, rank - 1, col);
-    whole[g] = col + V <= length;  // then i + V <= count too
-    if (!whole[g]) continue;
+    if (col + V > length) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[g][j] = i + j < count ? src[source_at<I>(i + j, rank, layout)] : T(0);
+      continue;
+    }
     const T* p = src + source_at<I>(row, rank - 1, layout) + int64_t(col) * step;
     if constexpr (UNIT) {
       v[g] = *reinterpret_cast<const Vec*>(p);
@@ -114,12 +118,14 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ 
     }
   }
 #pragma unroll
-  for (int g = 0; g < kGroups; ++g) {
+  for (int g = 0; g < G; ++g) {
     const I i = at[g];
-    if (whole[g]) {
+    if (i + V <= count) {
       *reinterpret_cast<Vec*>(dst + i) = v[g];
-    } else if (i < count) {
-      for (int j = 0; j < V && i + j < count; ++j) dst[i + j] = src[source_at<I>(i + j, rank, layout)];
+    } else {
+#pragma unroll
+      for (int j = 0; j < V; ++j)
+        if (i + j < count) dst[i + j] = v[g][j];
     }
   }
 }
@@ -263,6 +269,22 @@ int transposed_axis(int rank, const int64_t* shape, const int64_t* strides, int 
   return best;
 }
 
+template <typename T, int V, int G>
+void run_gather_rows(hp_ctx* ctx, const T* src, T* dst, int64_t count, int rank, Strided& layout) {
+  const int64_t grid = hp::ceil_div(count, 256 * V * G);
+  hp::require(grid <= hp::kMaxGrid, "gather too large for one launch");
+  const bool unit = layout.strides[rank - 1] == 1 || layout.shape[rank - 1] == 1;
+  // 31-bit indices, the overhang of the last workgroup included.
+  if (grid * 256 * V * G <= INT32_MAX) {
+    for (int d = 0; d < rank; ++d) layout.div[d] = make_divider(layout.shape[d]);
+    if (unit) gather_rows_kernel<T, V, true, uint32_t, G><<<grid, 256, 0, ctx->stream>>>(src, dst, uint32_t(count), rank, layout);
+    else gather_rows_kernel<T, V, false, uint32_t, G><<<grid, 256, 0, ctx->stream>>>(src, dst, uint32_t(count), rank, layout);
+  } else {
+    if (unit) gather_rows_kernel<T, V, true, int64_t, G><<<grid, 256, 0, ctx->stream>>>(src, dst, count, rank, layout);
+    else gather_rows_kernel<T, V, false, int64_t, G><<<grid, 256, 0, ctx->stream>>>(src, dst, count, rank, layout);
+  }
+}
+
 template <typename T, int V>
 void run_gather(hp_ctx* ctx, const void* src_, void* dst_, int64_t count, int64_t offset, int rank, Strided layout) {
   const T* src = static_cast<const T*>(src_) + offset;
@@ -303,18 +325,15 @@ void run_gather(hp_ctx* ctx, const void* src_, void* dst_, int64_t count, int64_
     layout.strides[0] = 1;
     rank = 1;
   }
-  const int64_t grid = hp::ceil_div(count, 256 * V * kGroups);
-  hp::require(grid <= hp::kMaxGrid, "gather too large for one launch");
-  const bool unit = layout.strides[rank - 1] == 1 || layout.shape[rank - 1] == 1;
-  // 31-bit indices, the overhang of the last workgroup included.
-  if (grid * 256 * V * kGroups <= INT32_MAX) {
-    for (int d = 0; d < rank; ++d) layout.div[d] = make_divider(layout.shape[d]);
-    if (unit) gather_rows_kernel<T, V, true, uint32_t><<<grid, 256, 0, ctx->stream>>>(src, dst, uint32_t(count), rank, layout);
-    else gather_rows_kernel<T, V, false, uint32_t><<<grid, 256, 0, ctx->stream>>>(src, dst, uint32_t(count), rank, layout);
-  } else {
-    if (unit) gather_rows_kernel<T, V, true, int64_t><<<grid, 256, 0, ctx->stream>>>(src, dst, count, rank, layout);
-    else gather_rows_kernel<T, V, false, int64_t><<<grid, 256, 0, ctx->stream>>>(src, dst, count, rank, layout);
-  }
+  // Runs per thread: one where every run crosses (every seventh column of
+  // 3000000 x 11 float32: 25.9 us, 27.7 with two), four where 8-byte words
+  // of a run are 32 bytes apart or more (300000 x 15 float64, transposed: 72 us
+  // against 80 with two; 1000000 x 4 20.5 against 22.4), else two (columns 1 to 9 of 3000000 x 11 float64: 88.7
+  // us against 92 with four).
+  const int64_t step = layout.strides[rank - 1] < 0 ? -layout.strides[rank - 1] : layout.strides[rank - 1];
+  if (layout.shape[rank - 1] < V) run_gather_rows<T, V, 1>(ctx, src, dst, count, rank, layout);
+  else if (sizeof(T) == 8 && step >= 4) run_gather_rows<T, V, 4>(ctx, src, dst, count, rank, layout);
+  else run_gather_rows<T, V, 2>(ctx, src, dst, count, rank, layout);
 }
 
 uint4 replicate(uint64_t bits, int elem_bytes) {

@@ -49,15 +49,13 @@ def test_gathers_match_numpy_strides(hip, name, dtype):
     np.testing.assert_array_equal(p.asnumpy(got).view(raw.dtype), want)
 
 
-@pytest.mark.parametrize("count", [2**31 - 4096, 2**31 - 4095, 2**31 - 2])
-def test_gathers_at_the_largest_arrays(hip, count):
-    # The last workgroup's overhang passes 31 bits from 2^31 - 4095 elements on:
-    # 64-bit indices there, 32-bit ones up to it. One row of 256, 167 or 331
-    # elements, read again and again.
-    length = next(n for n in range(331, 1, -1) if count % n == 0)
+# (elements, row): the last workgroup's overhang (2048 elements) passes 31 bits
+# from 2^31 - 2047 elements on: 64-bit indices there, 32-bit ones before.
+@pytest.mark.parametrize("count,length", [(2**31 - 2048, 384), (2**31 - 2046, 14), (2**31 - 2, 331)])
+def test_gathers_at_the_largest_arrays(hip, count, length):
     host = np.random.default_rng(count).integers(0, 2, length).astype(np.bool_)
     source = p.asarray(host, backend=hip)
-    shape = (count // length, length)
+    shape = (count // length, length)  # one row, read again and again
     got = p.asnumpy(p.ndarray._wrap(hip.gather(source, shape, 0, (0, 1)), shape, host.dtype, hip))
     for rows in np.array_split(got, 64):
         assert np.array_equal(rows, np.broadcast_to(host, rows.shape))
