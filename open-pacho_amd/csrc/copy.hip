@@ -255,18 +255,33 @@ int64_t grid_for(int64_t work, int64_t per_block) {
 }
 
 // The axis whose src stride makes a transposing gather worth its LDS tile, or
-// -1: the axis of the smallest stride is not the innermost one, steps of the
-// innermost axis are in other lines (>= 128 bytes apart) while those of this
-// one are in the same (<= 16 bytes), and both are long enough to use a good
-// part of a tile.
+// -1. It is the axis of the smallest stride (<= 16 bytes: neighbours share
+// lines) and not the innermost one, whose steps are lines apart or nearly
+// (kApart). A tile costs what a whole one costs however much of it is used, so
+// the share of its kTile x kTile elements decides, against rows that read each
+// line anew unless the caches keep it: they do for blocks of up to some hundred
+// lines (`rows`, the innermost extent), hardly for a thousand. Measured, us in
+// rows / tiles, 64 MB each: float32 blocks of 32 x 32 (a quarter used) 22 / 32,
+// 48 x 32 23 / 24, 48 x 64 34 / 20; 16 lanes (a quarter) x 256 36 / 31, x 4096
+// 78 / 30, x 500000 149 / 31; 12 lanes (0.19) x 256 36 / 39, x 1024 46 / 39;
+// float64 16 x 16 (0.06; 205 MB) 72 / 257, 16 lanes x 256 34 / 27, 12 lanes x 256
+// 30 / 33, x 1024 84 / 33. Runs that cross row ends cost rows a little: 33 x 33
+// (0.27; 20000 float64) 85 / 73. A last tile of a few rows writes parts of lines:
+// 65 x 65 (0.26; 20000 float64) 327 / 519, 80 x 80 (0.39) 509 / 550.
 int transposed_axis(int rank, const int64_t* shape, const int64_t* strides, int elem_bytes) {
-  constexpr int64_t kShortest = 16;
+  const int64_t kApart = elem_bytes >= 4 ? 48 : 128;
   const auto bytes = [&](int d) { return (strides[d] < 0 ? -strides[d] : strides[d]) * elem_bytes; };
-  if (rank < 2 || shape[rank - 1] < kShortest || bytes(rank - 1) < 128) return -1;
+  if (rank < 2 || bytes(rank - 1) < kApart) return -1;
   int best = -1;
   for (int d = 0; d < rank - 1; ++d)
-    if (shape[d] >= kShortest && bytes(d) > 0 && bytes(d) <= 16 && (best < 0 || bytes(d) < bytes(best))) best = d;
-  return best;
+    if (shape[d] > 1 && bytes(d) > 0 && bytes(d) <= 16 && (best < 0 || bytes(d) < bytes(best))) best = d;
+  if (best < 0) return -1;
+  const int64_t lanes = shape[best], rows = shape[rank - 1];
+  const auto share = [](int64_t n) { return double(n) / double(hp::ceil_div(n, kTile) * kTile); };
+  const bool sliver = rows > kTile && rows < 256 && (rows - 1) % kTile < 16;
+  const bool crossing = elem_bytes >= 4 && rows % (16 / elem_bytes) != 0;
+  const double least = sliver ? 0.45 : rows < 64 ? (crossing ? 0.25 : 1.0 / 3) : rows < 1024 ? 0.23 : 0.18;
+  return share(lanes) * share(rows) >= least ? best : -1;
 }
 
 template <typename T, int V, int G>

@@ -33,6 +33,15 @@ FORMS = {
     "repeated-inner": (77, 0, (77, 90), (1, 0)),
     "rank8": (2**8, 0, (2,) * 8, tuple(2 ** (7 - (3 * d) % 8) for d in range(8))),
     "one": (9, 8, (), ()),
+    # Either side of the shares of a tile that decide for or against tiles.
+    "third": (32 * 43, 0, (32, 43), (1, 32)),
+    "below a third": (32 * 42, 0, (32, 42), (1, 32)),
+    "quarter": (16 * 256, 0, (16, 256), (1, 16)),
+    "below a quarter": (3 * 14 * 250, 0, (3, 14, 250), (14 * 250, 1, 14)),
+    "fifth": (12 * 1152, 0, (12, 1152), (1, 12)),
+    "below a fifth": (11 * 1100, 0, (11, 1100), (1, 11)),
+    "sliver": (5 * 100 * 65, 0, (5, 100, 65), (6500, 1, 100)),
+    "wide sliver": (5 * 128 * 65, 0, (5, 128, 65), (8320, 1, 128)),
 }
 
 
