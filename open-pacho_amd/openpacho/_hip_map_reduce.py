@@ -87,6 +87,10 @@ class _Mapped:
         """(index, C type) of the leaves read in one of these ways."""
         return [(k, source_.ctype(self.leaves[k].dtype)) for k, a in enumerate(self.access) if a in kinds]
 
+    def bytes_read(self):
+        """Of the leaves that every element reads anew."""
+        return prod(self.shape) * sum(self.leaves[k].dtype.itemsize for k, _ in self.reads("full", "any"))
+
     def combine(self, left, right):
         return source_._combine(self.operation, self.acc_dtype, left, right)
 
@@ -227,14 +231,24 @@ def _rows(m):
 GROUPS_PER_CU = 2
 LEAST_ROWS = 16
 MOST_PARTIAL_BYTES = 8 << 20
+# A reduction of at most so many bytes and rows does without partials.
+ONE_LAUNCH_BYTES = 16 << 20
+ONE_LAUNCH_ROWS = 8192
 
 
-def _column_plan(outer, reduced, inner, width, acc_bytes, unit=1):
+def _column_plan(outer, reduced, inner, width, acc_bytes, unit=1, read=None):
     """(groups of `width` columns a workgroup spans, column blocks, rows per
     step, rows per chunk, chunks). Of the ways to cut a row into equal blocks
     of at least 16 groups (256 bytes of 4-byte columns), a multiple of `unit`,
     the one that leaves the fewest threads without a column, the widest of
-    equals."""
+    equals. Where that would leave partials of an array of few rows and bytes
+    (`read`, None for an array of any size), blocks of a few columns take all
+    rows in one launch instead: its lines come from the caches when neighbours
+    read them again, and a second launch costs more than that (float32, us a
+    call with partials / without: 300 x 17 15.5 / 7.4, 1000 x 1001 17.1 / 8.3,
+    8000 x 64 16.5 / 8.0, 4000 x 1024 17.0 / 8.3; past the limits 4000 x 4096
+    17.6 / 19.0, 8000 x 1001 17.0 / 17.2). The fewer the rows the wider the
+    blocks, about 16 rows a thread, from 16 bytes of columns on."""
     groups = -(-inner // width)
     best, fewest = None, -(-groups // BLOCK)
     for blocks in range(fewest, min(max(fewest, groups // 16), fewest + 32) + 1):
@@ -248,7 +262,13 @@ def _column_plan(outer, reduced, inner, width, acc_bytes, unit=1):
     chunks = min(chunks, max(1, MOST_PARTIAL_BYTES // (outer * inner * acc_bytes)))
     rows = max(-(-reduced // chunks), LEAST_ROWS * step)
     rows = -(-rows // step) * step
-    return across, blocks, step, rows, -(-reduced // rows)
+    chunks = -(-reduced // rows)
+    if chunks > 1 and reduced <= ONE_LAUNCH_ROWS and read is not None and read <= ONE_LAUNCH_BYTES:
+        least = -(-16 // (width * acc_bytes))
+        across = min(groups, max(least, min(8, LEAST_ROWS * BLOCK // reduced)))
+        step = BLOCK // across
+        return across, -(-groups // across), step, -(-reduced // step) * step, 1
+    return across, blocks, step, rows, chunks
 
 
 def _folded_rows(m, width):
@@ -260,7 +280,7 @@ def _folded_rows(m, width):
     columns does it without partials."""
     if m.inner % width == 0 or m.reads("reduced"):
         return 1, False
-    if _column_plan(m.outer, m.reduced, m.inner, 1, m.acc_dtype.itemsize)[4] == 1:
+    if _column_plan(m.outer, m.reduced, m.inner, 1, m.acc_dtype.itemsize, read=m.bytes_read())[4] == 1:
         return 1, False
     for period, least in ((8 * width, 64), (width, 16)):
         rows = period // gcd(m.inner, period)
@@ -327,7 +347,8 @@ def _columns(m):
     inner, total = folded * m.inner, m.reduced * m.inner
     reduced = -(-m.reduced // folded)
     across, blocks, step, rows, chunks = _column_plan(
-        m.outer, reduced, inner, width, m.acc_dtype.itemsize, 8 if lines_whole else 1
+        m.outer, reduced, inner, width, m.acc_dtype.itemsize, 8 if lines_whole else 1,
+        m.bytes_read() if folded == 1 else None,
     )
     grid = m.outer * chunks * blocks
     lambdas, given = m.lambdas("full", "reduced", "outer", "inner", "one")

@@ -57,6 +57,9 @@ def test_mapped_reductions_are_exact_on_small_integers(hip, shape, axes, index):
 # row, at the edges of the rule (64 long rows of lines, 16 of vectors), batched.
 FOLDED = [((rows, 5), (0,)) for rows in (64, 816, 817, 1024, 1027, 2047, 2048, 2049, 2079, 2080)]
 FOLDED += [((4 * 1024 + 3, 1025), (0,)), ((3001, 14), (0,)), ((40001, 6), (0,)), ((3, 2051, 7), (1,)), ((2, 30, 71, 9), (1, 2))]
+# Past the rows or the bytes of one launch without partials.
+FOLDED += [((rows, 5), (0,)) for rows in (8192, 8193, 8223, 8224)] + [((rows, 2051), (0,)) for rows in (2047, 2048, 2079)]
+FOLDED += [((9001, 14), (0,)), ((3, 8195, 7), (1,)), ((2, 130, 71, 9), (1, 2))]
 
 
 @pytest.mark.gpu
@@ -78,8 +81,8 @@ def test_folded_rows_are_exact_on_small_integers(hip, shape, axes, dtype):
 # Rows of each shape that become one, by the rule: as many as start on a line
 # where 64 long rows are left, on a vector where 16 are; one where single columns
 # need no partials, and where rows are whole vectors. (4- and 8-byte elements)
-FOLDS = [(1, 1), (1, 1), (4, 2), (4, 16), (4, 16), (4, 16), (32, 16), (32, 16), (32, 16), (32, 16)]
-FOLDS += [(32, 16), (16, 1), (16, 1), (32, 16), (32, 16)]
+FOLDS = [(1, 1)] * 10 + [(32, 16), (1, 1), (16, 1), (1, 1), (1, 1)]
+FOLDS += [(1, 1), (32, 16), (32, 16), (32, 16), (4, 16), (32, 16), (32, 16), (16, 1), (32, 16), (32, 16)]
 
 
 @pytest.mark.parametrize("case,folds", list(zip(FOLDED, FOLDS, strict=True)))
@@ -99,7 +102,8 @@ def test_folded_rows_start_on_lines_or_vectors_and_their_plans_cover_them(case, 
     inner, reduced = folded * m.inner, -(-m.reduced // folded)
     assert inner * dtype.itemsize % (128 if lines else 16) == 0 and reduced >= (64 if lines else 16)
     assert m.outer * inner * dtype.itemsize <= MOST_PARTIAL_BYTES
-    across, blocks, step, rows, chunks = _column_plan(m.outer, reduced, inner, width, dtype.itemsize, 8 if lines else 1)
+    unit = 8 if lines else 1
+    across, blocks, step, rows, chunks = _column_plan(m.outer, reduced, inner, width, dtype.itemsize, unit)
     assert across * step <= BLOCK and (blocks - 1) * across * width < inner <= blocks * across * width
     assert rows % step == 0 and (chunks - 1) * rows < reduced <= chunks * rows
 
@@ -143,10 +147,12 @@ def test_column_plans_cover_every_element_once(width):
     rng = np.random.default_rng(width)
     sizes = [1, 2, 3, 15, 16, 17, 255, 256, 257, 1025, 4096, 100003]
     for outer, reduced, inner in [(int(a), int(b), int(c)) for a, b, c in rng.choice(sizes, (400, 3))]:
-        across, blocks, step, rows, chunks = _column_plan(outer, reduced, inner, width, 8)
-        groups = -(-inner // width)
-        assert across * step <= BLOCK and (blocks - 1) * across < groups <= blocks * across
-        assert rows % step == 0 and (chunks - 1) * rows < reduced <= chunks * rows
+        for read in (None, outer * reduced * inner * 8):
+            across, blocks, step, rows, chunks = _column_plan(outer, reduced, inner, width, 8, read=read)
+            groups = -(-inner // width)
+            assert across * step <= BLOCK and (blocks - 1) * across < groups <= blocks * across
+            assert rows % step == 0 and (chunks - 1) * rows < reduced <= chunks * rows
+            assert chunks == 1 or read is None or reduced > 8192 or read > 16 << 20
 
 
 @pytest.mark.parametrize("shape,axes", [((8, 100, 12), (1,)), ((8, 3, 12), (0, 2)), ((5, 8193), (1,))])
