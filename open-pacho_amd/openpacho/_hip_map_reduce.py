@@ -146,8 +146,9 @@ def _rows(m):
     pairs, then with the lane's accumulator; lanes meet in a butterfly and
     waves in LDS. Bound by HBM: full leaves are read in 16-byte loads at
     element alignment, with the nontemporal hint where a wave reads whole
-    lines of one row (16384 x 4000 float32: 45 against 50 us) and without it
-    where rows share lines (1200000 x 49: 45 against 73 us). Max of x * x over
+    lines of one row (16384 x 4000 float32: 45 against 50 us; `stream` below
+    for 8-byte elements) and without it where rows share lines (1200000 x 49:
+    45 against 73 us). Max of x * x over
     the rows of 65536 x 4001 float32: 170 us (6.2 TB/s). With an element per
     lane and load and a workgroup per row, the max over rows took 107 us at
     16384 x 4000 and 47 us at 68848 x 49; now 45 and 6 us."""
@@ -157,14 +158,20 @@ def _rows(m):
     vectors = m.reads("full", "reduced")
     constants = [f"const {t} s{k} = x{k}[{'o' if m.access[k] == 'outer' else '0'}];" for k, t in m.reads("outer", "one")]
     stride, in_flight = lanes * VECTOR, 4
-    stream = "true" if lanes >= 64 else "false"
+
+    def stream(k):
+        # reduce.hip, streams(): of 8-byte leaves only those beyond the last
+        # cache whose rows start on lines.
+        size = m.leaves[k].dtype.itemsize
+        far = prod(m.leaves[k].shape) * size > 256_000_000 and m.reduced * size % 128 == 0
+        return "true" if lanes >= 64 and (size < 8 or far) else "false"
 
     def declare(u):
         return [f"{t} l{u}_{k}[{VECTOR}];" for k, t in vectors]
 
     def load(u):
         index = {"full": f"first + r + {u * stride}", "reduced": f"r + {u * stride}"}
-        return [f"pacho_loadu<{stream}>(x{k} + ({index[m.access[k]]}), l{u}_{k});" for k, t in vectors]
+        return [f"pacho_loadu<{stream(k)}>(x{k} + ({index[m.access[k]]}), l{u}_{k});" for k, t in vectors]
 
     def fold(u):
         def value(e):
