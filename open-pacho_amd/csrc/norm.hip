@@ -460,8 +460,6 @@ RowPlan plan_rows(hp_ctx* ctx, const T* x, int64_t outer, int64_t reduced) {
   if (reduced <= kShort) {
     plan.lanes = Traits<T>::width;  // load_chunk's last elements take a lane each
     while (plan.lanes < 64 && plan.lanes * 16 < reduced) plan.lanes *= 2;
-    plan.grid = hp::ceil_div(outer, kBlock / plan.lanes);
-    hp::require(plan.grid <= hp::kMaxGrid, "too many rows for one launch");
     return plan;
   }
   plan.vector = reinterpret_cast<uintptr_t>(x) % 16 == 0 && (reduced * int64_t(sizeof(T))) % 16 == 0 &&
@@ -487,8 +485,15 @@ void run_rows(hp_ctx* ctx, const RowPlan& plan, const T* x, T* out, int64_t oute
               Workspace ws) {
   const int64_t grid = plan.grid, chunks = plan.chunks;
   if (plan.lanes > 0) {
-    norm_short_kernel<T><<<grid, kBlock, 0, ctx->stream>>>(x, out, outer, reduced, plan.lanes);
-    hp::check_launch("norm_short");
+    // A launch takes fewer than 2^32 threads: 2^30 rows of one float32 would
+    // already be as many.
+    const int64_t per_group = kBlock / plan.lanes, most = (int64_t(1) << 23) * per_group;
+    for (int64_t o = 0; o < outer; o += most) {
+      const int64_t rows = outer - o < most ? outer - o : most;
+      norm_short_kernel<T><<<hp::ceil_div(rows, per_group), kBlock, 0, ctx->stream>>>(x + o * reduced, out + o, rows,
+                                                                                     reduced, plan.lanes);
+      hp::check_launch("norm_short");
+    }
     return;
   }
   const bool direct = plan.mode == kFinal || plan.mode == kWalk;

@@ -76,3 +76,14 @@ def test_short_rows_keep_squares_below_half_a_unit(hip, length, dtype):
     got = p.asnumpy(p.linalg.norm(p.asarray(host, backend=hip), axis=1))
     exact = np.linalg.norm(host.astype(np.longdouble), axis=1)
     np.testing.assert_allclose(got, exact.astype(np.float64), rtol=(4 + 2 + 6 + 1) / 4 * np.finfo(dtype).eps)
+
+
+@pytest.mark.parametrize("rows", [(1 << 29) + 3, (1 << 30) + 65])
+def test_more_short_rows_than_one_launch_takes(hip, rows):
+    # The norm of a single element is its absolute value.
+    x = p.random.default_rng(3, backend=hip).normal(0.0, 1.0, (rows, 1), dtype="float32")
+    norms = p.linalg.norm(x, axis=1)
+    apart = np.max(np.abs(norms - np.abs(x.reshape(rows))))
+    assert float(p.asnumpy(apart)) == 0
+    del x, apart
+    assert float(p.asnumpy(norms[-1:])[0]) > 0  # the last row was written
