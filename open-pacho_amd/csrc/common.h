@@ -113,8 +113,10 @@ inline void check_launch(const char* name) {
   }
 }
 
-// Grid dimension cap of a 1-D launch; kernels use grid-stride loops beyond it.
-constexpr int64_t kMaxGrid = int64_t(1) << 30;
+// Most workgroups of a 1-D launch of 256 threads each: a launch takes fewer
+// than 2^32 threads, and drops the workgroups past them without an error.
+constexpr int64_t kMaxGrid = (int64_t(1) << 24) - 1;
+constexpr int64_t kMaxThreads = (int64_t(1) << 32) - 1;
 
 inline size_t dtype_size(int dtype) {
   switch (dtype) {

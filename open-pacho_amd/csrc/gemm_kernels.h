@@ -1759,6 +1759,7 @@ void launch_split(hp_ctx* ctx, Whole whole, Cut cut, Fix fixup, int threads, con
   Split sp = plan_split(tm.total, hp::ceil_div(k, bk), ctx->compute_units, per_cu);
   sp.moved = moved;
   if (sp.dp_tiles > 0) {
+    hp::require(sp.dp_tiles <= hp::kMaxThreads / threads, "GEMM has too many tiles for one launch");
     whole<<<sp.dp_tiles, threads, 0, ctx->stream>>>(a, b, c, m, n, k, bd, tm, sp);
     hp::check_launch(name);
   }

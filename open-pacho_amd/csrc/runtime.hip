@@ -359,8 +359,8 @@ int hp_rtc_launch(hp_ctx* ctx, hp_kernel* kernel, int64_t grid, int block, int s
   return guarded([&] {
     hp::enter(ctx);
     require(kernel != nullptr && kernel->function != nullptr, "null kernel");
-    require(grid >= 0 && grid <= hp::kMaxGrid, "grid out of range");
     require(block > 0 && block <= 1024, "block out of range");
+    require(grid >= 0 && grid <= hp::kMaxThreads / block, "grid out of range: too many threads for one launch");
     if (grid == 0) return;
     HP_CHECK(hipModuleLaunchKernel(kernel->function, static_cast<unsigned>(grid), 1, 1,
                                    static_cast<unsigned>(block), 1, 1,
@@ -372,8 +372,8 @@ int hp_rtc_launch_packed(hp_ctx* ctx, hp_kernel* kernel, int64_t grid, int block
   return guarded([&] {
     hp::enter(ctx);
     require(kernel != nullptr && kernel->function != nullptr, "null kernel");
-    require(grid >= 0 && grid <= hp::kMaxGrid, "grid out of range");
     require(block > 0 && block <= 1024, "block out of range");
+    require(grid >= 0 && grid <= hp::kMaxThreads / block, "grid out of range: too many threads for one launch");
     require(bytes >= 0 && bytes <= 4096 && (args != nullptr || bytes == 0), "argument bytes out of range");
     if (grid == 0) return;
     size_t size = static_cast<size_t>(bytes);
