@@ -151,6 +151,41 @@ bool direct_serves(int64_t cus, int dtype, int64_t m, int64_t n, int64_t k, int6
   return tiles64 <= 1.5 * cus && work <= 2.2e9;
 }
 
+// Whether the staged kernels take a product of few K slices in less time than
+// `p`. A direct tile costs a start, a merge of four waves' accumulators and a
+// store, whatever K is: with one or two slices to a wave that is most of its
+// time, while a staged tile starts its stores after a slice or two. Times, us,
+// of rounds of one tile per compute unit: staged 128 x 128 in fp32 2.2 + 1.1 per
+// slice, 3.5 + 2.3 where one extent is shorter than the tile and 6 + 4 where
+// both are (4-byte loads); 256 x 128 in fp64 6 + 3.5 per slice, 4.3 with a K
+// edge. Direct 64 x 64 in fp32 1.4 + 1.4 per slice of a wave, an eighth more with
+// a K edge, smaller tiles 0.22 of it and the rest by area; 32 x 64 in fp64 2.6 +
+// 1.5, 0.1 and the rest by area. Fitted to 25 shapes in both types with K from 4
+// to 300 (staged | direct): 288 x (130 x 667 x 20) 61 | 107, 600 x (80 x 450 x 16)
+// 51 | 92, x 64 112 | 105, 2000 x (100 x 100 x 8) 80 | 94, x 32 116 | 94, 5606 x 426
+// x 25 10.4 | 12.7; fp64 290 x 3952 x 13 12 | 15, x 20 17 | 15, 288 x (130 x 667 x
+// 200) 429 | 537, x 300 643 | 612.
+bool staged_serves_few_slices(int64_t cus, int dtype, int64_t m, int64_t n, int64_t k, int64_t batch,
+                              const hpgemm::DirectPlan& p) {
+  const bool single = dtype == HP_F32;
+  if (p.splits > 1 || p.tiles <= cus || p.slices > (single ? 16 : 24)) return false;
+  const auto rounds = [&](int64_t tiles) { return double(hp::ceil_div(tiles, cus)); };
+  const double slices = double(p.slices), steps = double(hp::ceil_div(p.slices, 4));
+  const bool edge = k % 16 != 0;
+  double staged, direct;
+  if (single) {
+    const int cut = (m < 128) + (n < 128);
+    staged = cut == 0 ? 2.2 + 1.1 * slices : cut == 1 ? 3.5 + 2.3 * slices : 6 + 4 * slices;
+    // Three of its workgroups share a compute unit, so that part of a round takes part of its time.
+    staged *= 1.15 * std::max(1.0, double(hp::ceil_div(m, 128) * hp::ceil_div(n, 128) * batch) / double(cus));
+    direct = 1.4 * (1 + steps) * (edge ? 1.125 : 1.0) * (0.22 + 0.78 * p.fi * p.fj / 16.0);
+  } else {
+    staged = 1.05 * (6 + (edge ? 4.3 : 3.5) * slices) * rounds(hp::ceil_div(m, 256) * hp::ceil_div(n, 128) * batch);
+    direct = (2.6 + 1.5 * steps) * (0.1 + 0.9 * p.fi * p.fj / 8.0);
+  }
+  return staged < direct * rounds(p.tiles);
+}
+
 }  // namespace
 
 // Tile and K split by the time they would take: a compute unit works off its
@@ -197,7 +232,7 @@ hpgemm::DirectPlan hpgemm::direct_plan(int compute_units, int dtype, int64_t m, 
       }
     }
   }
-  return best;
+  return staged_serves_few_slices(compute_units, dtype, m, n, k, batch, best) ? DirectPlan{} : best;
 }
 
 using hp::guarded;

@@ -36,6 +36,20 @@ def test_large_and_whole_products_stay_staged():
     assert plan(np.float64, 512, 768, 1024, 64) is None and plan(np.float64, 4096, 4096, 4096) is None
 
 
+# (type, m, n, k, batch): few K slices in many tiles, either side of the rule.
+FEW_STAGED = [(np.float32, 130, 667, 20, 288), (np.float32, 80, 450, 8, 166), (np.float32, 255, 188, 96, 200)]
+FEW_STAGED += [(np.float32, 5606, 426, 25, 1), (np.float32, 100, 100, 8, 2000), (np.float32, 80, 450, 32, 600), (np.float32, 200, 40, 8, 400)]
+FEW_STAGED += [(np.float64, 290, 3952, 13, 1), (np.float64, 100, 100, 16, 128), (np.float64, 130, 667, 200, 288)]
+FEW_DIRECT = [(np.float32, 130, 667, 20, 4), (np.float32, 80, 450, 64, 600), (np.float32, 100, 100, 32, 2000)]
+FEW_DIRECT += [(np.float32, 9, 9, 4, 20000), (np.float32, 64, 64, 8, 8000), (np.float32, 20, 300, 20, 1500)]
+FEW_DIRECT += [(np.float64, 290, 3952, 20, 1), (np.float64, 130, 667, 300, 288), (np.float64, 64, 64, 16, 256)]
+
+
+def test_few_slices_in_many_tiles():
+    assert [case for case in FEW_STAGED if plan(*case)] == []
+    assert [case for case in FEW_DIRECT if not plan(*case)] == []
+
+
 def test_plans_refuse_what_is_no_product():
     with pytest.raises(ValueError):
         plan(np.int32, 4, 4, 4)
