@@ -377,10 +377,26 @@ def _columns(m):
     most = -(-rows // (batch * step))  # batches of a thread
     levels = most.bit_length() if m.operation == "sum" and m.acc_dtype.kind == "f" and most > LONGEST_CHAIN else 0
 
+    def within(j):
+        return f"r + {j * step} < whole"
+
+    def left_over():
+        """The loads of a batch that is not full."""
+        lines = []
+        for j in range(batch - 1):
+            lines += [f"{t} l{j}_{k}[{width}] = {{}};" for k, t in m.reads("full")] + [f"{t} l{j}_{k} = {{}};" for k, t in m.reads("reduced")]
+            at = f"first + r * {inner}LL + {j * step * inner}LL"
+            some = [f"pacho_loadu<{stream}>(x{k} + ({at}), l{j}_{k});" for k, _ in m.reads("full")]
+            some += [f"l{j}_{k} = x{k}[r + {j * step}];" for k, _ in m.reads("reduced")]
+            lines.append(f"if ({within(j)}) {{ {' '.join(some)} }}")
+        return lines
+
     def fold(count, into="acc"):
+        full = count == batch
         lines = []
         for v in range(width):
-            lines += ["{", *(f"  {m.acc} some{j} = {value(j, v)};" for j in range(count))]
+            some = (value(j, v) if full else f"{within(j)} ? {value(j, v)} : {m.identity}" for j in range(count))
+            lines += ["{", *(f"  {m.acc} some{j} = {one};" for j, one in enumerate(some))]
             apart = 1
             while apart < count:
                 for j in range(0, count - apart, 2 * apart):
@@ -431,9 +447,11 @@ def _columns(m):
       {FENCE}
       {_lines(fold(batch, "carry") + join if levels else fold(batch), 6)}
     }}
-    for (; r < whole; r += {step}) {{
-      {_lines(loads(0), 6)}
-      {_lines(fold(1), 6)}
+    if (r < whole) {{  // the rows left over, as one batch
+      {_lines(left_over(), 6)}
+      {FENCE}
+      {_lines(fold(batch - 1, "carry") + join if levels else fold(batch - 1), 6)}
+      while (r < whole) r += {step};
     }}
     if (r < end) {{
       for (int v = 0; v < {width}; ++v) {{
