@@ -12,9 +12,10 @@ Storage is an _Allocation (device pointer + capacity) from the library's
 stream-ordered pool. All work of a backend runs on its single stream, so an
 allocation may be returned while kernels that read it are still queued.
 Returned blocks of the pool's smallest size class (0-d results, short
-vectors) wait in a short host-side list for the next small request instead
-of crossing into the library twice; pool statistics, releases and close()
-hand that list back first. Operations never download or fall back
+vectors) and of its other power-of-two classes wait in short host-side lists
+for the next request instead of crossing into the library twice; pool
+statistics, releases, close() and a call that runs out of memory hand those
+lists back first. Operations never download or fall back
 to the CPU: a missing library or device raises BackendUnavailableError and a
 failing call raises.
 """
@@ -43,6 +44,7 @@ _SMALL_KEPT = 64
 # Blocks of the pool's power-of-two classes up to _KEPT_BLOCK wait on the host
 # too, at most _KEPT of each class (32 MiB in all), while the pool's limit is
 # far above that: a short operation's cost is its calls, and this saves two.
+# They go back when memory runs out (_again).
 _KEPT_BLOCK = 1 << 20
 _KEPT = 16
 _KEPT_POOL_LIMIT = 1 << 30
