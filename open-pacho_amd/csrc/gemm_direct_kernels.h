@@ -117,6 +117,7 @@ struct Tiles {
   int64_t tiles_m, tiles_n, per_batch, total;  // total over the batch
   int64_t slices, per_split;
   int64_t lda, ldb;
+  int64_t first;  // tile of this launch's first workgroup
 };
 
 template <typename T, int FI, int FJ, int DEPTH, bool TA, bool TB>
@@ -134,7 +135,8 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? 2 : 1) void direct_ke
   // Consecutive ids of one XCD (id % 8) take neighbouring tiles, in groups of
   // kGroupM tile rows.
   const uint32_t full = gridDim.x / 8 * 8;
-  const uint32_t id = blockIdx.x < full ? (blockIdx.x % 8) * (full / 8) + blockIdx.x / 8 : blockIdx.x;
+  const uint32_t at = blockIdx.x < full ? (blockIdx.x % 8) * (full / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int64_t id = t.first + at;
   const int64_t split = id / t.total;
   int64_t rest = id - split * t.total;
   const int64_t batch = rest / t.per_batch;
@@ -278,18 +280,21 @@ template <typename T, int FI, int FJ, int DEPTH>
 void launch(hp_ctx* ctx, const DirectPlan& plan, bool ta, bool tb, const T* a, const T* b, T* c, int64_t m, int64_t n,
             int64_t k, const BatchDesc& bd, int64_t batch) {
   Tiles t{plan.tiles_m, plan.tiles_n, plan.tiles_m * plan.tiles_n, plan.tiles, plan.slices, plan.per_split,
-          ta ? m : k, tb ? k : n};
-  const int64_t grid = plan.tiles * plan.splits, count = m * n * batch;
-  hp::require(grid <= hp::kMaxGrid, "GEMM has too many tiles for one launch");
+          ta ? m : k, tb ? k : n, 0};
+  const int64_t workgroups = plan.tiles * plan.splits, count = m * n * batch;
   T* target = plan.splits > 1 ? static_cast<T*>(hp::scratch_alloc(ctx, size_t(plan.splits) * count * sizeof(T))) : c;
+  // Batches of many small matrices pass what one launch takes.
+  for (; t.first < workgroups; t.first += hp::kMaxGrid) {
+    const int64_t grid = workgroups - t.first < hp::kMaxGrid ? workgroups - t.first : hp::kMaxGrid;
 #define PACHO_DIRECT(TA, TB) \
   direct_kernel<T, FI, FJ, DEPTH, TA, TB><<<grid, 64 * kWaves, 0, ctx->stream>>>(a, b, target, m, n, k, bd, t)
-  if (ta && tb) PACHO_DIRECT(true, true);
-  else if (ta) PACHO_DIRECT(true, false);
-  else if (tb) PACHO_DIRECT(false, true);
-  else PACHO_DIRECT(false, false);
+    if (ta && tb) PACHO_DIRECT(true, true);
+    else if (ta) PACHO_DIRECT(true, false);
+    else if (tb) PACHO_DIRECT(false, true);
+    else PACHO_DIRECT(false, false);
 #undef PACHO_DIRECT
-  hp::check_launch("gemm_direct");
+    hp::check_launch("gemm_direct");
+  }
   if (plan.splits == 1) return;
   add_splits_kernel<T><<<hp::ceil_div(count, 1024), 256, 0, ctx->stream>>>(target, c, count, plan.splits);
   hp::check_launch("gemm_add_splits");

@@ -188,9 +188,11 @@ template <typename T>
 void run_gemv(hp_ctx* ctx, const T* a, const T* x, const T* rhs, T* y, int64_t rows, int64_t inner) {
   const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   if (inner < 1024) {
-    const int64_t grid = hp::ceil_div(rows, 4);
-    hp::require(grid <= hp::kMaxGrid, "too many rows for one launch");
-    gemv_short_kernel<T><<<grid, kBlock, 0, ctx->stream>>>(a, x, rhs, y, rows, inner);
+    for (int64_t r = 0; r < rows; r += 4 * hp::kMaxGrid) {  // as many as one launch takes
+      const int64_t some = rows - r < 4 * hp::kMaxGrid ? rows - r : 4 * hp::kMaxGrid;
+      gemv_short_kernel<T><<<hp::ceil_div(some, 4), kBlock, 0, ctx->stream>>>(a + r * inner, x, rhs ? rhs + r : nullptr,
+                                                                            y + r, some, inner);
+    }
   } else {
     const int64_t grid = hp::ceil_div(rows, kRows);
     hp::require(grid <= hp::kMaxGrid, "too many rows for one launch");

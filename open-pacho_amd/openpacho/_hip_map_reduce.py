@@ -20,6 +20,7 @@ WAVES = BLOCK // 64
 # each load to its use and one is in flight at a time.
 FENCE = "__builtin_amdgcn_sched_barrier(0);"
 COMPUTE_UNITS = 256  # of the gfx950 parts these sources are compiled for
+MOST_WORKGROUPS = 2**24 - 1  # of BLOCK threads: a launch takes fewer than 2^32
 
 
 class MapReduce(tuple):
@@ -118,10 +119,18 @@ class _Mapped:
         given = [k for k, _ in self.reads(*kinds)]
         return self._lambda("mapped", given) + "\n  " + self._lambda("element", []), given
 
-    def kernel(self, body):
+    def kernel(self, body, workgroups=0):
+        """The kernel of `body`; with more `workgroups` than a launch takes, the
+        body (for workgroup `at`) in a loop over them."""
+        loop, close = "const unsigned at = blockIdx.x;", ""
+        if workgroups > MOST_WORKGROUPS:
+            loop = f"for (unsigned at = blockIdx.x; at < {workgroups}U; at += gridDim.x) {{"
+            close = "__syncthreads();  // the next one writes the same LDS\n}"
         return f"""{source_._PRELUDE}
 extern "C" __global__ __launch_bounds__({BLOCK}) void pacho_map_reduce({self.params}) {{
+{loop}
 {body}
+{close}
 }}
 """
 
@@ -425,7 +434,7 @@ def _columns(m):
   }}""" if step > 1 else ""
     body = f"""  __shared__ {m.acc} partial[{BLOCK * width if step > 1 else 1}];
   {lambdas}
-  const unsigned id = blockIdx.x < {grid // 8 * 8}U ? blockIdx.x % 8 * {grid // 8}U + blockIdx.x / 8 : blockIdx.x;
+  const unsigned id = at < {grid // 8 * 8}U ? at % 8 * {grid // 8}U + at / 8 : at;
   const unsigned block = id % {blocks}U, chunk = id / {blocks}U % {chunks}U;
   const long long o = id / {blocks * chunks}U;
   const int row = threadIdx.x / {across};
@@ -466,7 +475,10 @@ def _columns(m):
   if (active && row == 0) {{
     for (int v = 0; v < {width}; ++v) out[(o * {chunks}LL + chunk) * {inner}LL + col + v] = acc[v];
   }}"""
-    return MapReduce(m.kernel(body), m.outer * m.inner, chunks * folded, grid, (m.outer, chunks * folded, m.inner))
+    return MapReduce(
+        m.kernel(body, grid), m.outer * m.inner, chunks * folded, min(grid, MOST_WORKGROUPS),
+        (m.outer, chunks * folded, m.inner),
+    )
 
 
 def _any(m):
@@ -476,7 +488,7 @@ def _any(m):
     chunks = max(1, -(-reduced // CHUNK))
     body = f"""  __shared__ {m.acc} partial[{WAVES}];
   {m._lambda("element", [])}
-  const long long g = blockIdx.x;
+  const long long g = at;
   const long long o = g / {chunks}LL, chunk = g % {chunks}LL;
   const long long begin = chunk * {CHUNK}LL;
   const long long end = begin + {CHUNK}LL < {reduced}LL ? begin + {CHUNK}LL : {reduced}LL;
@@ -497,4 +509,5 @@ def _any(m):
     for (int w = 1; w < {WAVES}; ++w) total = {m.combine("total", "partial[w]")};
     out[g] = total;
   }}"""
-    return MapReduce(m.kernel(body), count, chunks, count * chunks, (count, chunks))
+    grid = count * chunks
+    return MapReduce(m.kernel(body, grid), count, chunks, min(grid, MOST_WORKGROUPS), (count, chunks))
